@@ -28,7 +28,9 @@
 //   QKV  - + bias, rounded, written head-major: Q,K [h][M][64] and V transposed [h][64][M]
 //          (replaces the reference's separate `layout` pass, kernels.cu:68-82);
 //   QKV_ROPE - QKV with rotate-half RoPE applied to Q and K in fp32 before the rounding.
+#include "gemm_burst.hpp"
 #include "kernels.hpp"
+#include "tiles.hpp"
 
 #include <atomic>
 #include <type_traits>
@@ -46,40 +48,6 @@ constexpr int BK = 64;
 // positions (measured on gfx950: swizzling by row % 8 instead leaves the two rows 8 apart on the
 // same banks, and rocprof's SQ_LDS_BANK_CONFLICT counts stalls for half of all LDS cycles).
 __device__ __forceinline__ int swz(int row) { return (row >> 1) & 7; }
-
-// Workgroup tile coordinates.  Workgroups are dealt to the 8 XCDs round-robin by linear dispatch
-// id, so consecutive ids run on different L2s.  When the workgroup count allows, the logical index
-// is laid out instead so that each XCD gets one contiguous share, decoded split-major: with split-K
-// an XCD works on whole K-slices (or an equal part of one) and fetches only those slices of both
-// operands.  Inside a slice, tiles are walked so the operand that is larger in HBM is fetched into
-// one L2 once: with many rows (A larger), groups of 4 tile rows with the column index outer; with
-// fewer rows than columns (B, the weights, larger), whole tile columns one after another.
-// Coordinates of logical tile `id` (0 .. nx ny nz - 1): the workgroup with linear dispatch id `id`
-// in the order above.
-__device__ __forceinline__ void tile_of(int id, int nx, int ny, int nz, bool rows_major, int* x, int* y, int* z) {
-  const int per_z = nx * ny, total = per_z * nz;
-  if (total % 8) {
-    *x = id % nx;
-    *y = (id / nx) % ny;
-    *z = id / per_z;
-    return;
-  }
-  const int l = (id % 8) * (total / 8) + id / 8;
-  *z = l / per_z;
-  const int t = l - *z * per_z;
-  if (rows_major) {
-    constexpr int G = 4;
-    const int group = t / (G * nx), first = group * G, size = min(G, ny - first), in = t - group * G * nx;
-    *y = first + in % size;
-    *x = in / size;
-  } else {
-    *x = t / ny;
-    *y = t - *x * ny;
-  }
-}
-__device__ __forceinline__ void tile_coords(int nx, int ny, int nz, bool rows_major, int* x, int* y, int* z) {
-  tile_of(blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z), nx, ny, nz, rows_major, x, y, z);
-}
 
 // Bytes of LDS the epilogue stages through: one 32 x 36 fp32 (or 32 x 40 16-bit) region per wave.
 constexpr int kEpilogueStageBytes = 32 * 36 * 4;
@@ -1063,6 +1031,7 @@ struct TileDef {
   bool ring;
   bool m16 = false;  // ring with 16x16x32 MFMAs (row-major and head-major epilogues without RoPE)
   bool persist = false;  // ring looping over tiles, one workgroup per CU (16-bit epilogues)
+  int burst = -1;        // variant of the few-row kernel (gemm_burst.hip)
   int threads() const { return 64 * wm * wn; }
 };
 // Tile menu; the planner picks per problem.  Ids are part of the op-level ABI (tests sweep them).
@@ -1109,8 +1078,12 @@ constexpr TileDef kTiles[] = {
     // Persistent form of tile 19 (gemm_ring_persist_kernel): a workgroup per CU walks the tiles, its
     // operand stream running on from one tile into the next.
     {256, 256, 2, 4, 0, 64, 5, true, false, true},  // 26
+    // 27 onwards: the few-row kernel (gemm_burst.hip).
+#define LAYA_BURST(V, BM, BN, WM, WN, KG, SL, S) {BM, BN, WM * KG, WN, 0, 0, 0, false, false, false, V},
+    LAYA_BURST_TILES
+#undef LAYA_BURST
 };
-constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
+[[maybe_unused]] constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 
 constexpr size_t lds_bytes(const TileDef& d) {
   return d.pf     ? static_cast<size_t>(2) * (d.bm + d.bn) * BK * 2
@@ -1118,20 +1091,22 @@ constexpr size_t lds_bytes(const TileDef& d) {
                   : static_cast<size_t>(d.st) * (d.bm + d.bn) * d.bk * 2;
 }
 
-// Compute units of the current device (the persistent tiles' grid), queried once per device.
-int device_cus() {
-  static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  int v = cache[dev].load(std::memory_order_relaxed);
-  if (v <= 0 && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-    cache[dev].store(v, std::memory_order_relaxed);
-  return v;
-}
+}  // namespace
+
+// The kernels of one epilogue are compiled in one translation unit each (LAYA_GEMM_EPI names it;
+// seven in parallel), the planner and the launcher in one more (LAYA_GEMM_EPI undefined).
+template <typename T, Epi E>
+hipError_t gemm_launch_t(const GemmArgs& a, int tile, hipStream_t stream);
+template <typename T, Epi E>
+hipError_t gemm_prepare_t();
+int gemm_device_cus();  // compute units of the current device (the persistent tiles' grid)
+
+#ifdef LAYA_GEMM_EPI
 
 template <typename T, Epi E>
-hipError_t launch_t(const GemmArgs& a, int tile, hipStream_t stream) {
+hipError_t gemm_launch_t(const GemmArgs& a, int tile, hipStream_t stream) {
   const TileDef& d = kTiles[tile];
+  if (d.burst >= 0) return launch_burst(a, E, std::is_same<T, f16>::value ? DType::F16 : DType::BF16, d.burst, stream);
   const dim3 grid(a.N / d.bn, (a.M + d.bm - 1) / d.bm, a.splits), block(d.threads());
   const size_t lds = lds_bytes(d);
   switch (tile) {
@@ -1174,7 +1149,7 @@ hipError_t launch_t(const GemmArgs& a, int tile, hipStream_t stream) {
       if constexpr (E == Epi::F32 || E == Epi::QKV_ROPE) {
         return hipErrorInvalidValue;
       } else {
-        const int cus = device_cus();
+        const int cus = gemm_device_cus();
         if (cus <= 0) return hipErrorInvalidDevice;
         const dim3 pgrid(min(static_cast<long long>(grid.x) * grid.y * grid.z, static_cast<long long>(cus)));
         LAYA_LAUNCH((gemm_ring_persist_kernel<T, E>), pgrid, block, lds, stream, a);
@@ -1190,7 +1165,7 @@ hipError_t launch_t(const GemmArgs& a, int tile, hipStream_t stream) {
 }
 
 template <typename T, Epi E>
-hipError_t set_lds_attr() {
+hipError_t gemm_prepare_t() {
   hipError_t e = hipSuccess;
 #define LAYA_ATTR(ID, ...)                                                                              \
   if (e == hipSuccess)                                                                                \
@@ -1226,15 +1201,35 @@ hipError_t set_lds_attr() {
   return e;
 }
 
+template hipError_t gemm_launch_t<f16, Epi::LAYA_GEMM_EPI>(const GemmArgs&, int, hipStream_t);
+template hipError_t gemm_launch_t<bf16, Epi::LAYA_GEMM_EPI>(const GemmArgs&, int, hipStream_t);
+template hipError_t gemm_prepare_t<f16, Epi::LAYA_GEMM_EPI>();
+template hipError_t gemm_prepare_t<bf16, Epi::LAYA_GEMM_EPI>();
+
+#else
+
+// Queried once per device.
+int gemm_device_cus() {
+  static std::atomic<int> cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  int v = cache[dev].load(std::memory_order_relaxed);
+  if (v <= 0 && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+    cache[dev].store(v, std::memory_order_relaxed);
+  return v;
+}
+
+namespace {
+
 template <typename T>
 hipError_t set_lds_all() {
-  hipError_t e = set_lds_attr<T, Epi::F32>();
-  if (e == hipSuccess) e = set_lds_attr<T, Epi::HALF>();
-  if (e == hipSuccess) e = set_lds_attr<T, Epi::GELU>();
-  if (e == hipSuccess) e = set_lds_attr<T, Epi::QKV>();
-  if (e == hipSuccess) e = set_lds_attr<T, Epi::QKV_ROPE>();
-  if (e == hipSuccess) e = set_lds_attr<T, Epi::RELU>();
-  if (e == hipSuccess) e = set_lds_attr<T, Epi::GEGLU>();
+  hipError_t e = gemm_prepare_t<T, Epi::F32>();
+  if (e == hipSuccess) e = gemm_prepare_t<T, Epi::HALF>();
+  if (e == hipSuccess) e = gemm_prepare_t<T, Epi::GELU>();
+  if (e == hipSuccess) e = gemm_prepare_t<T, Epi::QKV>();
+  if (e == hipSuccess) e = gemm_prepare_t<T, Epi::QKV_ROPE>();
+  if (e == hipSuccess) e = gemm_prepare_t<T, Epi::RELU>();
+  if (e == hipSuccess) e = gemm_prepare_t<T, Epi::GEGLU>();
   return e;
 }
 
@@ -1246,8 +1241,9 @@ GemmTile gemm_tile(int id) { return GemmTile{kTiles[id].bm, kTiles[id].bn}; }
 hipError_t gemm_prepare() {
   hipError_t e = set_lds_all<bf16>();
   if (e == hipSuccess) e = set_lds_all<f16>();
+  if (e == hipSuccess) e = burst_prepare();
   // The persistent tile's grid reads the CU count at launch: query it here, before any capture.
-  if (e == hipSuccess && device_cus() <= 0) e = hipErrorInvalidDevice;
+  if (e == hipSuccess && gemm_device_cus() <= 0) e = hipErrorInvalidDevice;
   return e;
 }
 
@@ -1267,7 +1263,65 @@ bool gemm_operands_addressable(long long M, long long lda, long long N, long lon
   return M * lda * 2 < (1LL << 32) && N * ldb * 2 < (1LL << 32);
 }
 
-void gemm_plan(int M, int N, int K, Epi epi, DType t, int cus, int* tile, int* splits, bool rope, bool measured) {
+namespace {
+
+// Few rows (at most kFewRows): launches are a few microseconds of fixed cost, operand stream and
+// output, so a tile's time follows a + s L nk + r (R - 1) + o MB, where L is the most tiles a CU gets,
+// nk its 64-deep slabs per tile, R the rounds of workgroups (two per CU where LDS allows) and MB
+// the output's megabytes.  The constants are fits to graph replays over weights that are cold in
+// every cache (12 row counts of 16-512, 14 projections of widths 768 and 1,024; 7-10% rms): the
+// choice they make is 2% slower on average than the best tile measured, where the plan table and
+// the larger-M heuristic below were 32% slower (96 rows, us: QKV 6.6 -> 4.7, with RoPE 9.9 -> 4.9,
+// GELU up 7.2 -> 5.7, GeGLU up 6.6 -> 4.6, out 4.1 -> 3.5; 16-bit 768 x 3,072 20.6 -> 9.3).  An
+// fp32 split costs its consumer another partial to read (0.12 us), and splits stop where the
+// partials would pass 8 MB.
+constexpr int kFewRows = 512;
+constexpr int kFewRowDepth = 512;  // shallower products (widths below 512) were not measured
+struct FewRowCost {
+  int tile, per_cu;
+  bool rope;
+  float a, s, r, o;
+};
+constexpr FewRowCost kFewRowCosts[] = {
+    {27, 2, true, 2.85f, 0.114f, 1.12f, 0.195f}, {28, 1, true, 3.06f, 0.144f, 1.99f, 0.134f},
+    {29, 1, true, 3.01f, 0.182f, 2.07f, 0.140f}, {30, 1, true, 2.98f, 0.202f, 1.89f, 0.204f},
+    {31, 1, true, 2.91f, 0.263f, 1.58f, 0.216f}, {32, 1, true, 3.35f, 0.237f, 2.04f, 0.231f},
+    {33, 1, false, 3.16f, 0.344f, 1.61f, 0.252f}, {34, 1, true, 3.08f, 0.400f, 1.47f, 0.206f},
+    {14, 1, false, 2.94f, 0.254f, 1.42f, 0.267f}, {23, 1, false, 2.83f, 0.332f, 1.21f, 0.281f},
+    {24, 1, false, 2.69f, 0.392f, 1.10f, 0.262f},
+};
+
+void few_row_plan(int M, int N, int K, Epi epi, int cus, bool rope, int max_splits, int* tile, int* splits) {
+  const bool head_major = epi == Epi::QKV || epi == Epi::QKV_ROPE;
+  const long long nk = K / BK;
+  float best = -1.f;
+  for (const FewRowCost& c : kFewRowCosts) {
+    const TileDef& d = kTiles[c.tile];
+    if (N % d.bn || (rope && !c.rope) || (head_major && d.burst >= 0 && 64 % d.bn)) continue;
+    const long long tiles = static_cast<long long>((M + d.bm - 1) / d.bm) * (N / d.bn);
+    for (int z = 1; z <= (epi == Epi::F32 ? max_splits : 1); z *= 2) {
+      if (z > 1 && (nk < 2 * z || static_cast<long long>(M) * N * 4 * z > (8LL << 20))) break;
+      const long long work = tiles * z, rounds = (work + cus * c.per_cu - 1) / (cus * c.per_cu);
+      const float mb = static_cast<float>(M) * N * (epi == Epi::F32 ? 4 * z : 2) * 1e-6f;
+      const float t = c.a + c.s * static_cast<float>((work + cus - 1) / cus * ((nk + z - 1) / z)) +
+                      c.r * static_cast<float>(rounds - 1) + c.o * mb + (epi == Epi::F32 ? 0.12f * z : 0.f);
+      if (best < 0.f || t < best) {
+        best = t;
+        *tile = c.tile;
+        *splits = z;
+      }
+    }
+  }
+}
+
+}  // namespace
+
+void gemm_plan(int M, int N, int K, Epi epi, DType t, int cus, int* tile, int* splits, bool rope, bool measured,
+               bool few_rows, int max_splits) {
+  if (few_rows && M <= kFewRows && N % 64 == 0 && K >= kFewRowDepth) {
+    few_row_plan(M, N, K, epi, cus, rope, max_splits, tile, splits);
+    return;
+  }
   for (const PlanEntry& e : kPlans) {
     if (!measured) break;
     if (e.cus == cus && e.M == M && e.N == N && e.K == K && e.epi == static_cast<int>(epi) &&
@@ -1363,22 +1417,26 @@ hipError_t launch_gemm(const GemmArgs& args, Epi epi, DType t, int tile, hipStre
   // Persistent tiles: 16-bit outputs without RoPE, at least three 64-deep slabs per tile.
   if (td.persist && (epi == Epi::F32 || epi == Epi::QKV_ROPE || (a.K / BK) % a.splits || a.K / BK / a.splits < 3))
     return hipErrorInvalidValue;
-  if (epi == Epi::QKV_ROPE && (td.bn / td.wn) % 64) return hipErrorInvalidValue;
+  if (epi == Epi::QKV_ROPE && td.burst < 0 && (td.bn / td.wn) % 64) return hipErrorInvalidValue;
+  // The few-row kernel's head-major epilogues take tiles within one head.
+  if ((epi == Epi::QKV || epi == Epi::QKV_ROPE) && td.burst >= 0 && 64 % td.bn) return hipErrorInvalidValue;
   if ((epi == Epi::QKV || epi == Epi::QKV_ROPE) && a.M % 8) return hipErrorInvalidValue;  // V^T: runs of 8 tokens
   if (epi == Epi::GEGLU && (a.N % 32 || a.ldo * 2 < a.N)) return hipErrorInvalidValue;
   if (epi == Epi::F32 && a.splits != 1 && a.bias) return hipErrorInvalidValue;  // bias joins the sum later
   const bool h = t == DType::F16;
   switch (epi) {
-    case Epi::F32: return h ? launch_t<f16, Epi::F32>(a, tile, stream) : launch_t<bf16, Epi::F32>(a, tile, stream);
-    case Epi::HALF: return h ? launch_t<f16, Epi::HALF>(a, tile, stream) : launch_t<bf16, Epi::HALF>(a, tile, stream);
-    case Epi::GELU: return h ? launch_t<f16, Epi::GELU>(a, tile, stream) : launch_t<bf16, Epi::GELU>(a, tile, stream);
-    case Epi::QKV: return h ? launch_t<f16, Epi::QKV>(a, tile, stream) : launch_t<bf16, Epi::QKV>(a, tile, stream);
+    case Epi::F32: return h ? gemm_launch_t<f16, Epi::F32>(a, tile, stream) : gemm_launch_t<bf16, Epi::F32>(a, tile, stream);
+    case Epi::HALF: return h ? gemm_launch_t<f16, Epi::HALF>(a, tile, stream) : gemm_launch_t<bf16, Epi::HALF>(a, tile, stream);
+    case Epi::GELU: return h ? gemm_launch_t<f16, Epi::GELU>(a, tile, stream) : gemm_launch_t<bf16, Epi::GELU>(a, tile, stream);
+    case Epi::QKV: return h ? gemm_launch_t<f16, Epi::QKV>(a, tile, stream) : gemm_launch_t<bf16, Epi::QKV>(a, tile, stream);
     case Epi::QKV_ROPE:
-      return h ? launch_t<f16, Epi::QKV_ROPE>(a, tile, stream) : launch_t<bf16, Epi::QKV_ROPE>(a, tile, stream);
-    case Epi::RELU: return h ? launch_t<f16, Epi::RELU>(a, tile, stream) : launch_t<bf16, Epi::RELU>(a, tile, stream);
-    case Epi::GEGLU: return h ? launch_t<f16, Epi::GEGLU>(a, tile, stream) : launch_t<bf16, Epi::GEGLU>(a, tile, stream);
+      return h ? gemm_launch_t<f16, Epi::QKV_ROPE>(a, tile, stream) : gemm_launch_t<bf16, Epi::QKV_ROPE>(a, tile, stream);
+    case Epi::RELU: return h ? gemm_launch_t<f16, Epi::RELU>(a, tile, stream) : gemm_launch_t<bf16, Epi::RELU>(a, tile, stream);
+    case Epi::GEGLU: return h ? gemm_launch_t<f16, Epi::GEGLU>(a, tile, stream) : gemm_launch_t<bf16, Epi::GEGLU>(a, tile, stream);
   }
   return hipErrorInvalidValue;
 }
+
+#endif  // LAYA_GEMM_EPI
 
 }  // namespace laya

@@ -314,8 +314,8 @@ void destroy_slot(Engine& E, Slot* s) {
 constexpr int kBranch16Rows = kBatchedRows;
 
 // Launch plans of a slot of shape (m, b, k): GEMM tiles and split-K, attention kernel, head
-// splits.  Host arithmetic only (no allocation).
-void plan_slot(const Engine& E, Slot* s, int m, int b, int k) {
+// splits.  Host arithmetic only (no allocation).  max_splits bounds the few-row plans' split-K.
+void plan_slot(const Engine& E, Slot* s, int m, int b, int k, int max_splits = 8) {
   const LayaConfig& c = E.cfg;
   s->m = m;
   s->b = b;
@@ -324,30 +324,33 @@ void plan_slot(const Engine& E, Slot* s, int m, int b, int k) {
   const int d = c.width, f = c.intermediate;
   LAYA_REQUIRE(gemm_operands_addressable(m, std::max(f, 4 * d), std::max(3 * d, 4 * d), std::max(f, 4 * d)),
                "a shape class of " + std::to_string(m) + " packed rows exceeds the 4 GiB GEMM operand limit");
-  gemm_plan(m, 3 * d, d, Epi::QKV, E.mfma(), E.cus, &s->tile[0], &s->splits[0], E.modern);
-  gemm_plan(m, d, d, Epi::F32, E.mfma(), E.cus, &s->tile[1], &s->splits[1]);
+  auto plan = [&](int M, int N, int K, Epi epi, int* tile, int* splits, bool rope = false) {
+    gemm_plan(M, N, K, epi, E.mfma(), E.cus, tile, splits, rope, true, true, max_splits);
+  };
+  plan(m, 3 * d, d, Epi::QKV, &s->tile[0], &s->splits[0], E.modern);
+  plan(m, d, d, Epi::F32, &s->tile[1], &s->splits[1]);
   if (E.modern) {
-    gemm_plan(m, 2 * f, d, Epi::GEGLU, E.mfma(), E.cus, &s->tile[2], &s->splits[2]);
+    plan(m, 2 * f, d, Epi::GEGLU, &s->tile[2], &s->splits[2]);
   } else {
-    gemm_plan(m, f, d, Epi::GELU, E.mfma(), E.cus, &s->tile[2], &s->splits[2]);
+    plan(m, f, d, Epi::GELU, &s->tile[2], &s->splits[2]);
   }
-  gemm_plan(m, d, f, Epi::F32, E.mfma(), E.cus, &s->tile[3], &s->splits[3]);
+  plan(m, d, f, Epi::F32, &s->tile[3], &s->splits[3]);
   s->splits[0] = s->splits[2] = 1;
   if (m >= kBranch16Rows) {
     s->branch16 = true;
-    gemm_plan(m, d, d, Epi::HALF, E.mfma(), E.cus, &s->tile[1], &s->splits[1]);
-    gemm_plan(m, d, f, Epi::HALF, E.mfma(), E.cus, &s->tile[3], &s->splits[3]);
+    plan(m, d, d, Epi::HALF, &s->tile[1], &s->splits[1]);
+    plan(m, d, f, Epi::HALF, &s->tile[3], &s->splits[3]);
     s->splits[1] = s->splits[3] = 1;
   }
   const int R = s->L.R;
   if (E.modern) {  // head transformer layers: all rows, then the readout rows of the last one
-    gemm_plan(m, 3 * d, d, Epi::QKV, E.mfma(), E.cus, &s->htile[0], &s->hsplits[0]);
-    gemm_plan(m, d, d, Epi::F32, E.mfma(), E.cus, &s->htile[1], &s->hsplits[1]);
-    gemm_plan(m, 4 * d, d, Epi::RELU, E.mfma(), E.cus, &s->htile[2], &s->hsplits[2]);
-    gemm_plan(m, d, 4 * d, Epi::F32, E.mfma(), E.cus, &s->htile[3], &s->hsplits[3]);
-    gemm_plan(R, d, d, Epi::F32, E.mfma(), E.cus, &s->htile[4], &s->hsplits[4]);
-    gemm_plan(R, 4 * d, d, Epi::RELU, E.mfma(), E.cus, &s->htile[5], &s->hsplits[5]);
-    gemm_plan(R, d, 4 * d, Epi::F32, E.mfma(), E.cus, &s->htile[6], &s->hsplits[6]);
+    plan(m, 3 * d, d, Epi::QKV, &s->htile[0], &s->hsplits[0]);
+    plan(m, d, d, Epi::F32, &s->htile[1], &s->hsplits[1]);
+    plan(m, 4 * d, d, Epi::RELU, &s->htile[2], &s->hsplits[2]);
+    plan(m, d, 4 * d, Epi::F32, &s->htile[3], &s->hsplits[3]);
+    plan(R, d, d, Epi::F32, &s->htile[4], &s->hsplits[4]);
+    plan(R, 4 * d, d, Epi::RELU, &s->htile[5], &s->hsplits[5]);
+    plan(R, d, 4 * d, Epi::F32, &s->htile[6], &s->hsplits[6]);
     s->hsplits[0] = s->hsplits[2] = s->hsplits[5] = 1;
   }
   // Few 128-query tiles (batch-1 requests): split each tile's keys across waves instead of
@@ -1160,7 +1163,11 @@ int laya_predict_static(void* handle, const int32_t* host_packed, const LayaShap
                  "invalid shape class");
     Slot s;  // plans and views into the scratch; owns nothing
     plan_slot(*E, &s, m, b, k);
-    const size_t need = carve_slot(*E, &s, nullptr);
+    size_t need = carve_slot(*E, &s, nullptr);
+    if (need > kScratchBytes) {  // without the few-row plans' split-K partials it may still fit
+      plan_slot(*E, &s, m, b, k, 1);
+      need = carve_slot(*E, &s, nullptr);
+    }
     LAYA_REQUIRE(need <= kScratchBytes,
                  "shape class (" + std::to_string(m) + ", " + std::to_string(b) + ", " + std::to_string(k) +
                      ") needs " + std::to_string(need) + " bytes of device scratch; laya_predict_static holds " +
@@ -1378,7 +1385,9 @@ int laya_op_linear(const void* x, const void* w, const float* bias, void* out, i
                                                                                                     : Epi::GEGLU;
     int cus = 256;
     if (tile < 0) {
-      gemm_plan(M, N, K, epi, half_type(dtype16), cus, &tile, &splits, false, tile == -1);
+      // fp32 plans: the caller sums the split partials, so their number is the table's and heuristic's.
+      gemm_plan(M, N, K, epi, half_type(dtype16), cus, &tile, &splits, false, tile == -1,
+                tile == -1 && epi != Epi::F32);
       if (bias) splits = 1;
     }
     LAYA_REQUIRE(tile < gemm_tile_count(), "bad tile id");
@@ -1399,7 +1408,7 @@ int laya_op_qkv(const void* x, const void* w, const float* bias, void* q, void* 
     int splits = 1;
     const bool rope = rope_cos != nullptr;
     LAYA_REQUIRE(!rope || (rope_sin && positions), "RoPE needs cos, sin and positions");
-    if (tile < 0) gemm_plan(M, 3 * width, width, Epi::QKV, half_type(dtype16), 256, &tile, &splits, rope, tile == -1);
+    if (tile < 0) gemm_plan(M, 3 * width, width, Epi::QKV, half_type(dtype16), 256, &tile, &splits, rope, tile == -1, tile == -1);
     LAYA_REQUIRE(tile < gemm_tile_count(), "bad tile id");
     LAYA_REQUIRE(width % 64 == 0 && (3 * width) % gemm_tile(tile).bn == 0, "width does not fit the tile");
     LAYA_REQUIRE(M % 8 == 0, "rows must be a multiple of 8 (V^T is stored in runs of 8 tokens)");

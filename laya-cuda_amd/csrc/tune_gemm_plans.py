@@ -1,6 +1,7 @@
 """Regenerate gemm_plans.inc: measured (tile, split-K) launches for the batch-1 GEMM problems.
 
-For every encoder shape family below, every packed-row class up to 2,048 rows (the classes
+For every encoder shape family below, every packed-row class from 640 to 2,048 rows (fewer rows are
+planned by the library's cost model) (the classes
 laya_cuda.runtime rounds requests to) and both MFMA input types, each GEMM of the forward is timed
 through the op-level C ABI (laya_op_linear / laya_op_qkv) with every tile id and, for the fp32
 split-K epilogue, 1/2/4/8 splits, and also with the library's own heuristic plan (tile -2); the
@@ -37,12 +38,8 @@ FAMILIES = [("bert-768", 768, 3072, False), ("bert-1024", 1024, 4096, False), ("
 
 
 def row_classes(limit=2048):
-    """Packed-row classes of laya_cuda.runtime._round_rows up to `limit`."""
-    out, m = [], 32
-    while m <= limit:
-        out.append(m)
-        m += 32 if m < 256 else 64 if m < 512 else 128
-    return out
+    """Packed-row classes of laya_cuda.runtime._round_rows above the few-row bound, up to `limit`."""
+    return list(range(640, limit + 1, 128))
 
 
 def problems(d, f, modern):

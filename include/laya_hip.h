@@ -217,8 +217,8 @@ int laya_op_norm(float* residual, const float* branch, int splits, int64_t part_
  * splits > 1, bias then must be NULL), 1: 16-bit out, 2: 16-bit exact-GELU out, 3: 16-bit ReLU out,
  * 4: GeGLU, out[M][N/2] = gelu(gate) * value with w's rows in the resident GeGLU interleave
  * (32-row groups: 16 gate rows, then their 16 value rows).  tile -1 lets the planner choose tile
- * and splits (splits ignored): for 16-bit outputs of few rows its cost model, else the measured plan
- * table when it holds the problem, else the heuristic; tile -2 takes the heuristic alone (the baseline the plan table is measured against). */
+ * and splits (splits ignored): for 16-bit outputs by its cost model, for fp32 by the measured plan
+ * table when it holds the problem, else the heuristic; tile -2 takes the heuristic alone. */
 int laya_op_linear(const void* x, const void* w, const float* bias, void* out, int kind,
                    int dtype16, int M, int N, int K, int splits, int tile, void* stream);
 

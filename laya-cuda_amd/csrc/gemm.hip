@@ -32,6 +32,7 @@
 #include "kernels.hpp"
 #include "tiles.hpp"
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -85,13 +86,10 @@ __device__ __forceinline__ f32x4 acc_quad(const f32x16& v, int r4) {
 template <typename T, int BM, int BN, int WM, int WN, Epi E, bool kEarlyBias, bool L16 = false, typename Acc>
 __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, Acc (&acc)[BM / WM / 32][BN / WN / 32],
                                               const float4 (&early_bias)[kEarlyBias ? BN / WN / 32 : 1][4],
-                                              const int (&early_pos)[BM / WM / 32], int m0, int n0, int z,
+                                              const int (&early_pos)[BM / WM / (L16 ? 16 : 32)], int m0, int n0, int z,
                                               unsigned char* smem_raw, int lane, int wave) {
   constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
-  static_assert(!L16 || (E != Epi::GEGLU && E != Epi::QKV_ROPE && !kEarlyBias),
-                "the 16x16 accumulator order serves the row-major and head-major epilogues without RoPE");
   const int wm0 = (wave / WN) * WTM, wn0 = (wave % WN) * WTN;
-  const int lrow = lane & 31, kg = lane >> 5;
   const bool with_bias = (E != Epi::F32 || a.splits == 1) && a.bias;
   // Epilogue.  Element r of lane l in a 32x32 tile of C^T is output column 8*(r/4) + 4*(l/32) +
   // r%4 of output row l%32: a lane holds columns c..c+3 of one row for each r/4.  The bias joins in
@@ -109,33 +107,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, Acc (&acc)[BM /
     }
   };
   typedef typename Vec4<T>::type T4;
-  if constexpr (E == Epi::GEGLU) {
-    // Weight rows interleaved in 32-row groups (16 gate rows, then their 16 value rows), so a lane
-    // holds gate column c (r4 < 2) and its value column c + 16 (r4 + 2): out[f] = gelu(gate) *
-    // value, 16 features per 32 columns (the reference's activate mode 2).
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int row = m0 + wm0 + i * 32 + lrow;
-      if (row >= a.M) continue;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int fbase = ((n0 + wn0 + j * 32) >> 1) + 4 * kg;
-#pragma unroll
-        for (int r4 = 0; r4 < 2; ++r4) {
-          float gate[4], value[4];
-          take(i, j, r4, gate);
-          take(i, j, r4 + 2, value);
-          T4 h;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) h[e] = to_half<T>(gelu16(gate[e]) * value[e]);
-          *reinterpret_cast<T4*>(static_cast<T*>(a.out) + static_cast<long long>(row) * a.ldo + fbase + 8 * r4) = h;
-        }
-      }
-    }
-    return;
-  }
-
-  // Every other epilogue leaves through LDS, one 32x32 tile at a time in this wave's own region
+  // Epilogues leave through LDS, one 32x32 tile at a time in this wave's own region
   // (the main loop's buffers are free: its last barrier has passed): the lanes write their column
   // quads, then read back 16-byte chunks of whole row segments, so each store instruction covers
   // 16 rows x 64 B (16-bit) or 8 rows x 128 B (fp32) instead of 32 rows x 8-16 B.  V^T goes through
@@ -145,13 +117,9 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, Acc (&acc)[BM /
   typedef typename std::conditional<E == Epi::F32, float, T>::type S;
   S* stg = reinterpret_cast<S*>(smem_raw) + wave * 32 * SP;
   const int rbase = m0 + wm0;  // first output row of this wave
-  // Row-major 32x32 tile: lane values h[r4] = the column quad r4 (quad_row, quad_col); chunk
-  // (r, c) (tile row r, first column c) is stored at dst(row, c) when row = rbase + 32 i + r < M.
-  auto emit_rows = [&](int i, const auto (&h)[4], auto dst) {
-    typedef typename std::remove_cv<typename std::remove_reference<decltype(h[0])>::type>::type Q;
-#pragma unroll
-    for (int r4 = 0; r4 < 4; ++r4)
-      *reinterpret_cast<Q*>(stg + quad_row<L16>(lane, r4) * SP + quad_col<L16>(lane, r4)) = h[r4];
+  // The staged 32x32 tile of row tile i: chunk (r, c) (tile row r, first column c) is stored at
+  // dst(row, c) when row = rbase + 32 i + r < M.
+  auto flush_rows = [&](int i, auto dst) {
     constexpr int EPC = 16 / sizeof(S), CPR = 32 / EPC;  // elements per chunk, chunks per row
 #pragma unroll
     for (int t = 0; t < 32 * CPR / 64; ++t) {
@@ -161,8 +129,48 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, Acc (&acc)[BM /
       if (row < a.M) *reinterpret_cast<i32x4*>(dst(row, col)) = v;
     }
   };
+  // Row-major 32x32 tile: lane values h[r4] = the column quad r4 (quad_row, quad_col).
+  auto emit_rows = [&](int i, const auto (&h)[4], auto dst) {
+    typedef typename std::remove_cv<typename std::remove_reference<decltype(h[0])>::type>::type Q;
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4)
+      *reinterpret_cast<Q*>(stg + quad_row<L16>(lane, r4) * SP + quad_col<L16>(lane, r4)) = h[r4];
+    flush_rows(i, dst);
+  };
 
-  if constexpr (E == Epi::F32) {
+  if constexpr (E == Epi::GEGLU) {
+    // Weight rows interleaved in 32-row groups (16 gate rows, then their 16 value rows), so a lane
+    // holds gate column c (r4 < 2) and its value column c + 16 (r4 + 2): out[f] = gelu(gate) *
+    // value, 16 features per 32 columns (the reference's activate mode 2).  In the 16x16 order the
+    // gate quads are r4 = 0 and 2 (rows 0-15 and 16-31), each followed by its value quad.  Two column
+    // tiles fill a staged 32x32 tile of features; a wave with one column tile stores its quads directly.
+    T* const out = static_cast<T*>(a.out);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int f0 = (n0 + wn0 + j * 32) >> 1;  // first feature of this column tile
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int gq = L16 ? 2 * s : s, vq = L16 ? gq + 1 : s + 2;
+          const int r = quad_row<L16>(lane, gq), c = quad_col<L16>(lane, gq);
+          float gate[4], value[4];
+          take(i, j, gq, gate);
+          take(i, j, vq, value);
+          T4 h;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) h[e] = to_half<T>(gelu16(gate[e]) * value[e]);
+          if constexpr (TN % 2 == 0) {
+            *reinterpret_cast<T4*>(stg + r * SP + (j & 1) * 16 + c) = h;
+          } else {
+            const int row = rbase + i * 32 + r;
+            if (row < a.M) *reinterpret_cast<T4*>(out + static_cast<long long>(row) * a.ldo + f0 + c) = h;
+          }
+        }
+        if (TN % 2 == 0 && (j & 1))
+          flush_rows(i, [&](int row, int col) { return out + static_cast<long long>(row) * a.ldo + f0 - 16 + col; });
+      }
+  } else if constexpr (E == Epi::F32) {
     float* out = static_cast<float*>(a.out) + z * a.split_stride;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -184,20 +192,28 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, Acc (&acc)[BM /
     // accumulator before the single rounding: tiles j and j+1 hold dims d and d+32 of one head.  The
     // cos/sin values of this lane's rows (dims 8 r4 + 4 kg .. +3 of each row's position) are all
     // read before the first tile is emitted: one memory round trip instead of one per row tile.
+    // (The 256-row tiles in 16x16 order have no registers for all of them beside their accumulators
+    // and read one row tile's at a time.)
     constexpr bool rope = E == Epi::QKV_ROPE;
-    float4 rcos[rope ? TM : 1][4], rsin[rope ? TM : 1][4];
-    if constexpr (rope) {
+    constexpr int RT = L16 && TM > 2 ? 1 : TM;
+    float4 rcos[rope ? RT : 1][4], rsin[rope ? RT : 1][4];
+    auto load_rope = [&](int first) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
-          const size_t at = static_cast<size_t>(early_pos[i]) * 32 + 8 * r4 + 4 * kg;
+          const int p = L16 ? early_pos[2 * (first + i) + (r4 >> 1)] : early_pos[first + i];
+          const size_t at = static_cast<size_t>(p) * 32 + quad_col<L16>(lane, r4);
           rcos[i][r4] = *reinterpret_cast<const float4*>(a.rope_cos + at);
           rsin[i][r4] = *reinterpret_cast<const float4*>(a.rope_sin + at);
         }
-    }
+    };
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
+      if constexpr (rope) {
+        if (RT < TM) __builtin_amdgcn_sched_barrier(0);
+        if (i % RT == 0) load_rope(i);
+      }
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         const int col0 = n0 + wn0 + j * 32;
@@ -216,8 +232,8 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, Acc (&acc)[BM /
                 float v0[4], v1[4];
                 take(i, j, r4, v0);
                 take(i, j + 1, r4, v1);
-                const float c4[4] = {rcos[i][r4].x, rcos[i][r4].y, rcos[i][r4].z, rcos[i][r4].w};
-                const float s4[4] = {rsin[i][r4].x, rsin[i][r4].y, rsin[i][r4].z, rsin[i][r4].w};
+                const float c4[4] = {rcos[i % RT][r4].x, rcos[i % RT][r4].y, rcos[i % RT][r4].z, rcos[i % RT][r4].w};
+                const float s4[4] = {rsin[i % RT][r4].x, rsin[i % RT][r4].y, rsin[i % RT][r4].z, rsin[i % RT][r4].w};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                   lo[r4][e] = to_half<T>(v0[e] * c4[e] - v1[e] * s4[e]);
@@ -561,8 +577,8 @@ void gemm_pipe_kernel(GemmArgs a) {
 #pragma unroll
     for (int r4 = 0; r4 < 4; ++r4) early_bias[0][r4] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
-  int early_pos[TM];
-  load_early_pos<TM, E>(a, m0 + wm0 + (lane & 31), early_pos);
+  int early_pos[M16 ? 2 * TM : TM] = {};  // 16x16 MFMAs: no RoPE here
+  if constexpr (!M16) load_early_pos<TM, E>(a, m0 + wm0 + (lane & 31), early_pos);
   const unsigned lds_base = lds_address(smem_raw);
   auto issue_at = [&](int q, int kt, int base) {  // base: element offset of the load's LDS destination
     lds_load16_buffer(q < AG ? rsA : rsB, src[q], static_cast<unsigned>(kt) * BKS * 2,
@@ -1024,6 +1040,254 @@ void gemm_ring_persist_kernel(GemmArgs a) {
   }
 }
 
+// Batched tiles: the persistent ring with 16x16x32 MFMAs (tile 35).  The walk over tiles, the ring
+// of five half-slab buffers and the epilogue staged in the last slab's A buffer are those of
+// gemm_ring_persist_kernel; what differs is the main loop, which is laid out by hand in rows of four
+// MFMAs (one 16-row block of the wave's 128x64 against its four column blocks):
+//   * v_mfma_f32_16x16x32 streams 2.03 PFLOP/s from two waves per SIMD on random operands against
+//     1.71 for 32x32x16 (register-only streams);
+//   * a slab's eight direct loads per wave go out one per row, four before and four after the slab's
+//     barrier.  Issued together after the barrier they kept both waves of a SIMD in the load queue
+//     (64 loads of 16 address cycles each per CU and slab) while its matrix core was idle;
+//   * the A fragments have one register set: block i is read for the next k-step right after the row
+//     that used it, seven rows before its next use, and only the four B fragments are double-buffered.
+//     64 fragment registers instead of 96 leave room for the tile loop without spills;
+//   * the barrier sits two rows into the slab's last k-step, so the LDS reads it waits for are two
+//     rows old.
+template <typename T, Epi E>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_ring16_kernel(GemmArgs a) {
+  // RoPE runs one tile per workgroup: beside the tile loop its cos/sin rows and positions spilled.
+  constexpr bool kLoop = E != Epi::QKV_ROPE;
+  constexpr int BM = 256, BN = 256, WM = 2, WN = 4, NW = WM * WN, BKS = 64;
+  constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32, MB = WTM / 16, NB = WTN / 16;
+  constexpr int CPR = BKS / 8, RPI = 64 / CPR;
+  constexpr int AG = BM / RPI / NW, BG = BN / RPI / NW;
+  constexpr int HALFB = BM * BKS * 2;  // bytes of a ring buffer
+  static_assert(E != Epi::F32, "16-bit epilogues: their staging fits one ring buffer");
+  static_assert(MB == 8 && NB == 4 && AG == 4 && BG == 4, "the row schedule below");
+  constexpr int kWaitSlab = waitcnt_vm(AG);
+  constexpr int kWaitFirst = waitcnt_vm(AG + BG);
+  constexpr int kWaitAll = waitcnt_vm(0);
+  typedef typename Vec8<T>::type T8;
+
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm0 = (wave / WN) * WTM, wn0 = (wave % WN) * WTN;
+  const int r16 = lane & 15, kq = lane >> 4;
+
+  const int nx = a.N / BN, ny = (a.M + BM - 1) / BM, total = nx * ny;
+  const int G = gridDim.x;
+  const int n = a.K / BKS;  // slabs per tile (the launcher checks n >= 3)
+  int id = blockIdx.x;
+  if (id >= total) return;
+
+  // Operands through per-tile buffer resources based at the tile's first A row and first B row (see
+  // gemm_ring_persist_kernel): rows past M are outside the A resource and never stored.
+  const int lr = lane / CPR, pch = lane % CPR;
+  // Load q of a half is 64 rows further on: the same swizzle, so its distance goes into the scalar
+  // offset (the range check is on the sum) and each operand takes one offset register.
+  const int row0 = wave * RPI + lr;
+  const unsigned chunk = static_cast<unsigned>(pch ^ swz_k<BKS>(row0)) << 3;
+  const unsigned srcA = (static_cast<unsigned>(row0) * static_cast<unsigned>(a.lda) + chunk) * 2u;
+  const unsigned srcB = (static_cast<unsigned>(row0) * static_cast<unsigned>(a.ldb) + chunk) * 2u;
+  const unsigned stepA = NW * RPI * 2u * static_cast<unsigned>(a.lda), stepB = NW * RPI * 2u * static_cast<unsigned>(a.ldb);
+  auto res_a = [&](int m0) {
+    return buffer_resource(static_cast<const T*>(a.a) + static_cast<size_t>(m0) * a.lda,
+                           static_cast<unsigned>(static_cast<size_t>(a.M - m0) * a.lda * 2));
+  };
+  auto res_b = [&](int n0) {
+    return buffer_resource(static_cast<const T*>(a.b) + static_cast<size_t>(n0) * a.ldb,
+                           static_cast<unsigned>(static_cast<size_t>(a.N - n0) * a.ldb * 2));
+  };
+  auto decode = [&](int t, int& m0, int& n0) {
+    int tx, ty, tz;
+    tile_of(t, nx, ny, 1, a.rows_major, &tx, &ty, &tz);
+    n0 = tx * BN;
+    m0 = ty * BM;
+  };
+  const unsigned lds_base = lds_address(smem_raw);
+
+  int m0, n0;
+  decode(id, m0, n0);
+  i32x4 rsA = res_a(m0), rsB = res_b(n0);
+  int nid = id + G, nm0 = m0, nn0 = n0;
+  bool has_next = kLoop && nid < total;
+  if (has_next) decode(nid, nm0, nn0);
+  i32x4 nrsA = res_a(nm0), nrsB = res_b(nn0);
+
+  // Load q of the A (or B) half of stream slab `s` counted from this tile's first slab: this tile's
+  // slab s, the next tile's slab s - n, or (last tile) this tile's last slab again, never read.
+  auto issue = [&](bool isB, int q, int s, int buf) {
+    const bool next = s >= n && has_next;
+    const int kt = next ? s - n : min(s, n - 1);
+    lds_load16_buffer(isB ? (next ? nrsB : rsB) : (next ? nrsA : rsA), isB ? srcB : srcA,
+                      static_cast<unsigned>(kt) * BKS * 2 + q * (isB ? stepB : stepA),
+                      lds_base + static_cast<unsigned>(buf * HALFB + (wave + NW * q) * RPI * BKS * 2));
+  };
+
+  // The tile's bias for this lane's column quads and, with RoPE, its rows' positions: loaded at the
+  // tile's start, since vector memory operations complete in issue order.
+  float4 bias[TN][4];
+  int pos[MB];
+  auto load_tile_inputs = [&]() {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {  // quads r4 and r4 + 2 share their columns
+        bias[j][c] = a.bias ? *reinterpret_cast<const float4*>(a.bias + n0 + wn0 + j * 32 + quad_col<true>(lane, c))
+                            : make_float4(0.f, 0.f, 0.f, 0.f);
+        bias[j][c + 2] = bias[j][c];
+      }
+    if constexpr (E == Epi::QKV_ROPE) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i) pos[i] = a.positions[min(m0 + wm0 + i * 16 + r16, a.M - 1)];
+    }
+  };
+  load_tile_inputs();
+
+  // Fragment addresses: block row i is 16 rows = 2 KB further on, and the swizzle (row / 2) % 8 is
+  // the same for all of them.
+  const int frag0 = r16 * 128 + ((kq ^ (r16 >> 1)) << 4), frag1 = r16 * 128 + (((4 + kq) ^ (r16 >> 1)) << 4);
+  T8 fa[MB], fb[2][NB];
+  auto read_a = [&](int buf, int kk, int i) {
+    fa[i] = *reinterpret_cast<const T8*>(smem_raw + (buf * HALFB + wm0 * 128 + (kk ? frag1 : frag0)) + i * 2048);
+  };
+  auto read_b = [&](int buf, int kk, int j) {
+    fb[kk][j] = *reinterpret_cast<const T8*>(smem_raw + (buf * HALFB + wn0 * 128 + (kk ? frag1 : frag0)) + j * 2048);
+  };
+  f32x4 acc[MB][NB];
+  auto row = [&](int i, int kk) {  // weights as the MFMA's A operand: the accumulator holds C^T
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = mfma16(fb[kk][j], fa[i], acc[i][j]);
+  };
+  auto pin = [] { __builtin_amdgcn_sched_barrier(0); };
+  auto next_two = [](int buf) { return buf >= 3 ? buf - 3 : buf + 2; };
+  auto next_one = [](int buf) { return buf == 4 ? 0 : buf + 1; };
+
+  // The first k-step of slab `it`: its second k-step's fragments are read, and the A half of slab
+  // it + 2 goes into the fifth buffer (slab it - 1's B).
+  auto first_step = [&](int it, int abuf, int bbuf) {
+    const int free_buf = abuf == 0 ? 4 : abuf - 1;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      if (i < NB) read_b(bbuf, 1, i);
+      if (i % 2 == 0) issue(false, i / 2, it + 2, free_buf);
+      pin();
+      row(i, 0);
+      pin();
+      read_a(abuf, 1, i);
+    }
+    pin();
+    row(0, 1);
+    row(1, 1);
+    pin();
+    publish_stage<kWaitSlab>();
+    pin();
+  };
+  auto read_first = [&](int abuf, int bbuf) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) read_b(bbuf, 0, j);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) read_a(abuf, 0, i);
+  };
+
+  // Prologue: slabs 0 and 1 into buffers 0 .. 3.
+#pragma unroll
+  for (int h = 0; h < 4; ++h)
+#pragma unroll
+    for (int q = 0; q < AG; ++q) issue(h & 1, q, h / 2, h);
+  publish_stage<kWaitFirst>();
+  read_first(0, 1);
+  int abuf = 0;  // buffer of the current slab's A half; its B half is in the next one
+  for (;;) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int it = 0; it < n - 1; ++it) {
+      const int bbuf = next_one(abuf), nabuf = next_two(abuf), nbbuf = next_one(nabuf);
+      first_step(it, abuf, bbuf);
+      // The rest of the last k-step: the next slab's fragments, and the B half of slab it + 2 into
+      // this slab's A buffer.
+#pragma unroll
+      for (int i = 2; i < MB; ++i) {
+        if (i < 6) {
+          read_a(nabuf, 0, i - 2);
+          read_b(nbbuf, 0, i - 2);
+          issue(true, i - 2, it + 2, abuf);
+        } else if (i == 6) {
+          read_a(nabuf, 0, 4);
+          read_a(nabuf, 0, 5);
+        } else {
+          read_a(nabuf, 0, 6);
+        }
+        pin();
+        row(i, 1);
+        pin();
+      }
+      read_a(nabuf, 0, 7);
+      abuf = nabuf;
+    }
+    // The tile's last slab: its A buffer takes the epilogue's staging, so the B half that belongs
+    // there is issued after it.
+    const int bbuf = next_one(abuf), nabuf = next_two(abuf), nbbuf = next_one(nabuf);
+    first_step(n - 1, abuf, bbuf);
+#pragma unroll
+    for (int i = 2; i < MB; ++i) row(i, 1);
+    // Quad r4 of 32x32 region (i, j) is 16x16 block (2 i + r4 / 2, 2 j + r4 % 2) (quad_row/quad_col).
+    f32x16 out[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) out[i][j][4 * q + e] = acc[2 * i + (q >> 1)][2 * j + (q & 1)][e];
+    // An opaque copy of the lane keeps the epilogue's lane-dependent addresses out of the tile loop's
+    // registers (hoisted there they spilled, and every reload waits for the whole operand prefetch).
+    int elane = lane;
+    asm volatile("" : "+v"(elane));
+    if constexpr (E == Epi::QKV_ROPE) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i) asm volatile("" : "+v"(pos[i]));
+    }
+    if (!kLoop || !has_next) {
+      // The clamped loads of the last slabs may still be landing: drain them before the epilogue
+      // reuses LDS (and before the workgroup ends).
+      __builtin_amdgcn_s_waitcnt(kWaitAll);
+      __syncthreads();
+      gemm_epilogue<T, BM, BN, WM, WN, E, true, true>(a, out, bias, pos, m0, n0, 0, smem_raw, elane, wave);
+      return;
+    }
+    gemm_epilogue<T, BM, BN, WM, WN, E, true, true>(a, out, bias, pos, m0, n0, 0,
+                                                    smem_raw + static_cast<size_t>(abuf) * HALFB, elane, wave);
+    // Every wave's staging reads are done before the ring load below overwrites the buffer (the
+    // epilogue's global stores stay in flight).
+    __builtin_amdgcn_s_waitcnt(waitcnt_lgkm0_keep_vm());
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    m0 = nm0;
+    n0 = nn0;
+    rsA = nrsA;
+    rsB = nrsB;
+    nid += G;
+    has_next = nid < total;
+    if (has_next) {
+      decode(nid, nm0, nn0);
+      nrsA = res_a(nm0);
+      nrsB = res_b(nn0);
+    }
+    load_tile_inputs();
+#pragma unroll
+    for (int q = 0; q < BG; ++q) issue(true, q, 1, abuf);
+    read_first(nabuf, nbbuf);
+    abuf = nabuf;
+  }
+}
+
 struct TileDef {
   int bm, bn, wm, wn;
   int pf;      // >= 2: register-staged kernel with pf slabs in flight; 0: pipelined direct-to-LDS kernel
@@ -1082,6 +1346,7 @@ constexpr TileDef kTiles[] = {
 #define LAYA_BURST(V, BM, BN, WM, WN, KG, SL, S) {BM, BN, WM * KG, WN, 0, 0, 0, false, false, false, V},
     LAYA_BURST_TILES
 #undef LAYA_BURST
+    {256, 256, 2, 4, 0, 64, 5, true, true, true},  // 35: gemm_ring16_kernel
 };
 [[maybe_unused]] constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 
@@ -1156,6 +1421,18 @@ hipError_t gemm_launch_t(const GemmArgs& a, int tile, hipStream_t stream) {
       }
       break;
     }
+    case 35: {
+      if constexpr (E == Epi::F32) {
+        return hipErrorInvalidValue;
+      } else {
+        const int cus = gemm_device_cus();
+        if (cus <= 0) return hipErrorInvalidDevice;
+        const long long tiles = static_cast<long long>(grid.x) * grid.y;
+        const dim3 pgrid(E == Epi::QKV_ROPE ? tiles : min(tiles, static_cast<long long>(cus)));
+        LAYA_LAUNCH((gemm_ring16_kernel<T, E>), pgrid, block, lds, stream, a);
+      }
+      break;
+    }
 #undef LAYA_RING
 #undef LAYA_TILE
 #undef LAYA_PIPE
@@ -1196,6 +1473,9 @@ hipError_t gemm_prepare_t() {
   LAYA_ATTR(25, gemm_pipe_kernel<T, 128, 128, 4, 2, 64, 4, E, false>)
   if constexpr (E != Epi::F32 && E != Epi::QKV_ROPE) {
     LAYA_ATTR(26, gemm_ring_persist_kernel<T, E>)
+  }
+  if constexpr (E != Epi::F32) {
+    LAYA_ATTR(35, gemm_ring16_kernel<T, E>)
   }
 #undef LAYA_ATTR
   return e;
@@ -1265,46 +1545,57 @@ bool gemm_operands_addressable(long long M, long long lda, long long N, long lon
 
 namespace {
 
-// Few rows (at most kFewRows): launches are a few microseconds of fixed cost, operand stream and
-// output, so a tile's time follows a + s L nk + r (R - 1) + o MB, where L is the most tiles a CU gets,
-// nk its 64-deep slabs per tile, R the rounds of workgroups (two per CU where LDS allows) and MB
+// Plans by cost: a launch's time follows a + s L nk + r (R - 1) + o MB, where L is the most tiles a CU
+// gets, nk its 64-deep slabs per tile, R the rounds of workgroups (two per CU where LDS allows) and MB
 // the output's megabytes.  The constants are fits to graph replays over weights that are cold in
-// every cache (12 row counts of 16-512, 14 projections of widths 768 and 1,024; 7-10% rms): the
-// choice they make is 2% slower on average than the best tile measured, where the plan table and
-// the larger-M heuristic below were 32% slower (96 rows, us: QKV 6.6 -> 4.7, with RoPE 9.9 -> 4.9,
-// GELU up 7.2 -> 5.7, GeGLU up 6.6 -> 4.6, out 4.1 -> 3.5; 16-bit 768 x 3,072 20.6 -> 9.3).  An
-// fp32 split costs its consumer another partial to read (0.12 us), and splits stop where the
-// partials would pass 8 MB.
+// every cache: 14 projections of widths 768 and 1,024 at 12 row counts of 16-512, and 16 at 18 row
+// counts of 640-24,576 (6-12% rms).  Up to 512 rows the choice they make is 2% slower on average than
+// the best tile measured, above 1%, where the plan table with the larger-tile heuristic it
+// replaced was 32% and 13% slower (us: 96-row QKV 6.6 -> 4.7, with RoPE 9.9 -> 4.9; 1,008-row GELU
+// up 18.1 -> 13.1, GeGLU up 14.1 -> 10.0, 768 x 768 with fp32 output 9.2 -> 6.0).  An fp32 split costs
+// its consumer another partial to read (0.12 us per 512 rows), and splits stop where the partials
+// would pass 16 MB.
 constexpr int kFewRows = 512;
-constexpr int kFewRowDepth = 512;  // shallower products (widths below 512) were not measured
-struct FewRowCost {
+constexpr int kCostDepth = 512;  // shallower products (widths below 512) were not measured
+struct TileCost {
   int tile, per_cu;
-  bool rope;
   float a, s, r, o;
+  int max_slabs = 1 << 30;
 };
-constexpr FewRowCost kFewRowCosts[] = {
-    {27, 2, true, 2.85f, 0.114f, 1.12f, 0.195f}, {28, 1, true, 3.06f, 0.144f, 1.99f, 0.134f},
-    {29, 1, true, 3.01f, 0.182f, 2.07f, 0.140f}, {30, 1, true, 2.98f, 0.202f, 1.89f, 0.204f},
-    {31, 1, true, 2.91f, 0.263f, 1.58f, 0.216f}, {32, 1, true, 3.35f, 0.237f, 2.04f, 0.231f},
-    {33, 1, false, 3.16f, 0.344f, 1.61f, 0.252f}, {34, 1, true, 3.08f, 0.400f, 1.47f, 0.206f},
-    {14, 1, false, 2.94f, 0.254f, 1.42f, 0.267f}, {23, 1, false, 2.83f, 0.332f, 1.21f, 0.281f},
-    {24, 1, false, 2.69f, 0.392f, 1.10f, 0.262f},
+constexpr TileCost kFewRowCosts[] = {
+    {27, 2, 2.85f, 0.114f, 1.12f, 0.195f}, {28, 1, 3.06f, 0.144f, 1.99f, 0.134f}, {29, 1, 3.01f, 0.182f, 2.07f, 0.140f},
+    {30, 1, 2.98f, 0.202f, 1.89f, 0.204f}, {31, 1, 2.91f, 0.263f, 1.58f, 0.216f}, {32, 1, 3.35f, 0.237f, 2.04f, 0.231f},
+    {33, 1, 3.16f, 0.344f, 1.61f, 0.252f}, {34, 1, 3.08f, 0.400f, 1.47f, 0.206f}, {14, 1, 2.94f, 0.254f, 1.42f, 0.267f},
+    {23, 1, 2.83f, 0.332f, 1.21f, 0.281f}, {24, 1, 2.69f, 0.392f, 1.10f, 0.262f},
+};
+// Tile 21's two-stage pipeline falls behind with depth (15,088 x 768: 26.5 against the ring's 24.2 us at
+// K = 768 but 92 against 76 at 3,072), so it is kept to the depths its constants were fitted on.
+constexpr TileCost kCosts[] = {
+    {14, 1, 3.92f, 0.198f, 2.17f, 0.048f}, {31, 1, 3.45f, 0.252f, 2.08f, 0.019f}, {34, 1, 3.76f, 0.389f, 2.30f, 0.074f},
+    {23, 1, 3.70f, 0.274f, 2.00f, 0.127f}, {24, 1, 3.83f, 0.275f, 2.02f, 0.109f}, {16, 1, 4.20f, 0.271f, 1.88f, 0.386f},
+    {25, 1, 4.02f, 0.394f, 3.31f, 0.132f}, {18, 1, 4.47f, 0.401f, 3.59f, 0.114f}, {9, 1, 4.32f, 0.902f, 1.80f, 0.321f},
+    {8, 1, 4.38f, 0.907f, 2.10f, 0.288f},  {21, 1, 6.58f, 0.962f, 4.89f, 0.257f, 16}, {35, 1, 6.28f, 1.026f, 3.28f, 0.380f},
 };
 
-void few_row_plan(int M, int N, int K, Epi epi, int cus, bool rope, int max_splits, int* tile, int* splits) {
+template <size_t C>
+bool cost_plan(const TileCost (&costs)[C], int M, int N, int K, Epi epi, int cus, bool rope, int max_splits, int* tile,
+               int* splits) {
   const bool head_major = epi == Epi::QKV || epi == Epi::QKV_ROPE;
   const long long nk = K / BK;
   float best = -1.f;
-  for (const FewRowCost& c : kFewRowCosts) {
+  for (const TileCost& c : costs) {
     const TileDef& d = kTiles[c.tile];
-    if (N % d.bn || (rope && !c.rope) || (head_major && d.burst >= 0 && 64 % d.bn)) continue;
+    if (N % d.bn || nk > c.max_slabs) continue;
+    if (d.burst >= 0 ? head_major && 64 % d.bn : rope && (d.bn / d.wn) % 64) continue;
+    if (d.persist && epi == Epi::F32) continue;
     const long long tiles = static_cast<long long>((M + d.bm - 1) / d.bm) * (N / d.bn);
     for (int z = 1; z <= (epi == Epi::F32 ? max_splits : 1); z *= 2) {
-      if (z > 1 && (nk < 2 * z || static_cast<long long>(M) * N * 4 * z > (8LL << 20))) break;
+      if (z > 1 && (nk < 2 * z || static_cast<long long>(M) * N * 4 * z > (16LL << 20))) break;
       const long long work = tiles * z, rounds = (work + cus * c.per_cu - 1) / (cus * c.per_cu);
       const float mb = static_cast<float>(M) * N * (epi == Epi::F32 ? 4 * z : 2) * 1e-6f;
       const float t = c.a + c.s * static_cast<float>((work + cus - 1) / cus * ((nk + z - 1) / z)) +
-                      c.r * static_cast<float>(rounds - 1) + c.o * mb + (epi == Epi::F32 ? 0.12f * z : 0.f);
+                      c.r * static_cast<float>(rounds - 1) + c.o * mb +
+                      (epi == Epi::F32 ? 0.12f * z * static_cast<float>(std::max(M, 512)) / 512.f : 0.f);
       if (best < 0.f || t < best) {
         best = t;
         *tile = c.tile;
@@ -1312,16 +1603,17 @@ void few_row_plan(int M, int N, int K, Epi epi, int cus, bool rope, int max_spli
       }
     }
   }
+  return best >= 0.f;
 }
 
 }  // namespace
 
 void gemm_plan(int M, int N, int K, Epi epi, DType t, int cus, int* tile, int* splits, bool rope, bool measured,
-               bool few_rows, int max_splits) {
-  if (few_rows && M <= kFewRows && N % 64 == 0 && K >= kFewRowDepth) {
-    few_row_plan(M, N, K, epi, cus, rope, max_splits, tile, splits);
+               bool by_cost, int max_splits) {
+  if (by_cost && N % 64 == 0 && K >= kCostDepth &&
+      (M <= kFewRows ? cost_plan(kFewRowCosts, M, N, K, epi, cus, rope, max_splits, tile, splits)
+                     : cost_plan(kCosts, M, N, K, epi, cus, rope, max_splits, tile, splits)))
     return;
-  }
   for (const PlanEntry& e : kPlans) {
     if (!measured) break;
     if (e.cus == cus && e.M == M && e.N == N && e.K == K && e.epi == static_cast<int>(epi) &&
@@ -1413,9 +1705,9 @@ hipError_t launch_gemm(const GemmArgs& args, Epi epi, DType t, int tile, hipStre
   if (epi == Epi::QKV && a.rope_cos) epi = Epi::QKV_ROPE;
   // RoPE needs both halves of a head in one lane: wave tiles of 64-column multiples.
   const TileDef& td = kTiles[tile];
-  if (td.m16 && (epi == Epi::QKV_ROPE || epi == Epi::GEGLU)) return hipErrorInvalidValue;
-  // Persistent tiles: 16-bit outputs without RoPE, at least three 64-deep slabs per tile.
-  if (td.persist && (epi == Epi::F32 || epi == Epi::QKV_ROPE || (a.K / BK) % a.splits || a.K / BK / a.splits < 3))
+  if (td.m16 && !td.persist && (epi == Epi::QKV_ROPE || epi == Epi::GEGLU)) return hipErrorInvalidValue;
+  // Persistent tiles: 16-bit outputs (tile 26 without RoPE), at least three 64-deep slabs per tile.
+  if (td.persist && (epi == Epi::F32 || (epi == Epi::QKV_ROPE && !td.m16) || (a.K / BK) % a.splits || a.K / BK / a.splits < 3))
     return hipErrorInvalidValue;
   if (epi == Epi::QKV_ROPE && td.burst < 0 && (td.bn / td.wn) % 64) return hipErrorInvalidValue;
   // The few-row kernel's head-major epilogues take tiles within one head.

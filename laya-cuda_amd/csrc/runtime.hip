@@ -314,7 +314,7 @@ void destroy_slot(Engine& E, Slot* s) {
 constexpr int kBranch16Rows = kBatchedRows;
 
 // Launch plans of a slot of shape (m, b, k): GEMM tiles and split-K, attention kernel, head
-// splits.  Host arithmetic only (no allocation).  max_splits bounds the few-row plans' split-K.
+// splits.  Host arithmetic only (no allocation).  max_splits bounds the cost model's split-K.
 void plan_slot(const Engine& E, Slot* s, int m, int b, int k, int max_splits = 8) {
   const LayaConfig& c = E.cfg;
   s->m = m;
@@ -1164,7 +1164,7 @@ int laya_predict_static(void* handle, const int32_t* host_packed, const LayaShap
     Slot s;  // plans and views into the scratch; owns nothing
     plan_slot(*E, &s, m, b, k);
     size_t need = carve_slot(*E, &s, nullptr);
-    if (need > kScratchBytes) {  // without the few-row plans' split-K partials it may still fit
+    if (need > kScratchBytes) {  // without the cost model's split-K partials it may still fit
       plan_slot(*E, &s, m, b, k, 1);
       need = carve_slot(*E, &s, nullptr);
     }

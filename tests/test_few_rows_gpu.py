@@ -1,4 +1,4 @@
-"""The few-row GEMM (csrc/gemm_burst.hip): every tile and epilogue at the edges of its tiles, stages
+"""The few-row GEMM (csrc/gemm_burst.hip) and the 16x16x32 ring (csrc/gemm.hip, tile 35): every tile and epilogue at the edges of its tiles, stages
 and K splits, and the planner's choice around its row bound, against 64-bit products of the same
 16-bit operands.
 
@@ -126,3 +126,52 @@ def test_planned_tiles_around_the_row_bound(gpu, M):
         close(out, ref + bias.double(), "f16", K)
     # N that no 64-wide tile divides stays refused, whatever the few-row tiles' width.
     assert lib.laya_op_linear(p(x), p(w), None, p(out), 1, _lib.F16, M, 32, 64, 1, -1, stream()) != 0
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(1, 256, 192), (300, 768, 576), (16421, 2048, 192), (30000, 768, 320)])
+def test_ring_of_sixteen_wide_mfmas(gpu, kind, M, N, K):
+    """Tile 35, the persistent 256x256 ring with 16x16x32 MFMAs: one tile, partial row tiles, the
+    three-slab minimum, and several tiles per workgroup (520 and 354 on 256 CUs), every 16-bit
+    row-major epilogue."""
+    t = torch()
+    lib = _lib.load()
+    x, w, bias, _ = operands(gpu, kind, M, N, K)
+    ref = t.mm(x.float(), w.float().t()).double()  # fp32 product of 64-bit-exact terms: within 1e-6 sqrt(K)
+    groups = ref.view(M, N // 32, 2, 16)
+    for epilogue, b, want in ((1, bias, ref + bias), (2, bias, t.nn.functional.gelu(ref + bias)),
+                              (3, bias, t.relu(ref + bias)),
+                              (4, None, (t.nn.functional.gelu(groups[:, :, 0]) * groups[:, :, 1]).reshape(M, -1))):
+        out = t.full(want.shape, float("nan"), dtype=half(kind), device=gpu)
+        _lib.check(lib.laya_op_linear(p(x), p(w), p(b), p(out), epilogue, code(kind), M, N, K, 1, 35, stream()))
+        close(out, want, kind, K)
+    out32 = t.zeros((M, N), device=gpu)
+    assert lib.laya_op_linear(p(x), p(w), None, p(out32), 0, code(kind), M, N, K, 1, 35, stream()) != 0  # 16-bit only
+    assert lib.laya_op_linear(p(x), p(w), None, p(out), 1, code(kind), M, N, 128, 1, 35, stream()) != 0  # two slabs
+
+
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("M,width", [(8, 256), (1000, 768), (16424, 1024)])
+def test_ring_of_sixteen_wide_mfmas_head_major(gpu, M, width, rope):
+    t = torch()
+    lib = _lib.load()
+    heads = width // 64
+    x, w, bias, _ = operands(gpu, "f16", M, 3 * width, width)
+    ref = t.mm(x.float(), w.float().t()).double()
+    g = t.Generator(device=gpu).manual_seed(3)
+    angle = t.rand((700, 32), generator=g, device=gpu) * 6
+    cos, sin = angle.cos().contiguous(), angle.sin().contiguous()
+    pos = t.randint(0, 700, (M,), generator=g, device=gpu, dtype=t.int32)
+    q, k, vt = (t.full((M * width,), float("nan"), dtype=t.float16, device=gpu) for _ in range(3))
+    _lib.check(lib.laya_op_qkv(p(x), p(w), p(bias), p(q), p(k), p(vt), p(cos) if rope else None,
+                               p(sin) if rope else None, p(pos) if rope else None, _lib.F16, M, width, 35, stream()))
+    wq, wk, wv = ((ref + bias)[:, i * width:(i + 1) * width].reshape(M, heads, 64).transpose(0, 1) for i in range(3))
+    if rope:
+        c, s = cos[pos.long()].double(), sin[pos.long()].double()
+
+        def rotate(v):
+            return t.cat([v[..., :32] * c - v[..., 32:] * s, v[..., 32:] * c + v[..., :32] * s], -1)
+        wq, wk = rotate(wq), rotate(wk)
+    close(q.view(heads, M, 64), wq, "f16", width)
+    close(k.view(heads, M, 64), wk, "f16", width)
+    close(vt.view(heads, 64, M), wv.transpose(1, 2), "f16", width)

@@ -385,15 +385,22 @@ __device__ __forceinline__ void attention_shared(const AttnArgs& a) {
   publish_stage<waitcnt_vm(0)>();
   // Waves past the tile's last row (the short last tile of a sequence) stage keys with the others
   // but skip the block math: in ragged batches that is a fifth of the query slots.
-  const bool active = row0 + wave * 32 < row1;
+  const int wq0 = row0 + uwave * 32;  // this wave's first query
+  const bool active = wq0 < row1;
+  // On local layers the wave's 32 queries see at most 160 of the up to 384 keys its tile stages: it skips
+  // the other blocks, and masks only those that reach past what every one of its queries sees.
+  const int wlast = min(wq0 + 31, row1 - 1);
+  const int wlo = local ? max(start, wq0 - a.window) : start, whi = local ? min(kend, wlast + a.window + 1) : kend;
+  const int all_lo = local ? max(start, wlast - a.window) : start;
+  const int all_hi = local ? min(kend, wq0 + a.window + 1) : kend;
   // Block j from buffer cur (a constant in each copy of the step, so the fragment reads keep fixed
   // addresses) while block j+1 streams into the other buffer.
   auto step = [&](int j, auto cur_c) {
     constexpr int cur = decltype(cur_c)::value;
     const int kb = klo + j * KB;
     if (j + 1 < nkb) kv_load_direct<T, NT>(K, Vt, a.m, kb + KB, ldsK[cur ^ 1], ldsV[cur ^ 1], tid, uwave);
-    if (active)
-      attend_block<T>(cur ? frag1 : frag0, qf, o, mrow, lsum, kb, local || kb + KB > kend, qlo, qhi, lane);
+    if (active && kb < whi && kb + KB > wlo)
+      attend_block<T>(cur ? frag1 : frag0, qf, o, mrow, lsum, kb, kb < all_lo || kb + KB > all_hi, qlo, qhi, lane);
     publish_stage<waitcnt_vm(0)>();
   };
   for (int j = 0; j < nkb; j += 2) {

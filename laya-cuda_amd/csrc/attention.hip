@@ -423,6 +423,194 @@ __device__ __forceinline__ void attention_shared(const AttnArgs& a) {
     }
 }
 
+// Eight-wave tiles, global layers: two four-wave workgroups per 256-query tile, each wave running one
+// block ahead of itself.  In attention_shared a wave's MFMAs (16 per block, 314 ns at the rate random
+// operands allow) and its softmax (about 100 VALU instructions and 32 exponentials, 299 ns) follow
+// each other, and the barrier of every block lines the waves of a SIMD up in the same phase: 64 x
+// 1,024 tokens ran at their sum.  Here, while the softmax of block j runs, the same wave's matrix
+// instructions are the scores of block j + 1 and the products of block j - 1 with V, which do not
+// depend on it, and no block needs its maximum first (below).  64 x 1,024 tokens, 16 heads: 346 -> 340 us;
+// the ragged 32-request batch's attention gains more (the 128-query workgroups leave no idle waves):
+// 4.96 -> 4.88 ms per forward.  What bounds it now is power: copies without the loads run 291 us, and
+// the MFMA stream alone lowers the clock to 1.6 GHz (19.6 ns per 32x32x16, 161 us in all).
+template <typename T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void attention_ahead_kernel(AttnArgs a) {
+  typedef typename Vec8<T>::type T8;
+  typedef typename Vec4<T>::type T4;
+  int tile, head;
+  if (a.n_tiles) {
+    const int used = min(*a.n_tiles, a.max_tiles) * 2;
+    if (!work_item_used(a.max_tiles * 2, a.heads, used, &tile, &head)) return;
+  } else {
+    work_item(a.max_tiles * 2, a.heads, &tile, &head);
+  }
+  const int4 td = reinterpret_cast<const int4*>(a.tiles)[tile >> 1];
+  const int row0 = td.x + (tile & 1) * 128, row1 = min(td.y, row0 + 128), start = td.z, len = td.w;
+  if (row0 >= row1) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ld = a.heads * 64;
+  T* out = static_cast<T*>(a.out);
+  if (len < 0) {
+    zero_rows(out, ld, head, row0, row1, tid, 256);
+    return;
+  }
+  const int kend = start + len, nkb = (len + KB - 1) / KB;
+  const int ql = lane & 31, g = lane >> 5;
+  const int q = row0 + wave * 32 + ql;
+  const bool qin = q < row1, qvalid = qin && q < kend;
+  const size_t plane = static_cast<size_t>(head) * a.m * 64;
+  // K and V^T through buffer resources of this head's planes: a lane's offset in a block is the same for
+  // every block.  Keys past the end of the slot read zeros (K) or the next head dim's first keys and zeros
+  // past the last one's (V^T): they lie past the end of every sequence, and their probabilities are 0.
+  const unsigned bytes = static_cast<unsigned>(static_cast<size_t>(a.m) * 128);
+  const i32x4 rsK = buffer_resource(static_cast<const T*>(a.k) + plane, bytes);
+  const i32x4 rsV = buffer_resource(static_cast<const T*>(a.vt) + plane, bytes);
+  const unsigned row_bytes = static_cast<unsigned>(a.m) * 2u;
+  unsigned srcK, srcV;
+  {
+    const int r = tid >> 3, lu = (tid & 7) ^ kvswz(r);  // rows r and r + 32 of a block
+    srcK = static_cast<unsigned>(kperm(r)) * 128u + lu * 16u;
+    srcV = static_cast<unsigned>(r) * row_bytes + lu * 16u;
+  }
+
+  __shared__ __align__(16) T sk[2][KB * 64];
+  __shared__ __align__(16) T sv[2][KB * 64];
+  const unsigned ldsK[2] = {lds_address(sk[0]), lds_address(sk[1])};
+  const unsigned ldsV[2] = {lds_address(sv[0]), lds_address(sv[1])};
+  auto load_k = [&](int kb, int buf) {
+#pragma unroll
+    for (unsigned i = 0; i < 2; ++i)
+      lds_load16_buffer(rsK, srcK, (static_cast<unsigned>(kb) + 32u * i) * 128u, ldsK[buf] + (wave + 4u * i) * 1024u);
+  };
+  auto load_v = [&](int kb, int buf) {
+#pragma unroll
+    for (unsigned i = 0; i < 2; ++i)
+      lds_load16_buffer(rsV, srcV, static_cast<unsigned>(kb) * 2u + i * 32u * row_bytes, ldsV[buf] + (wave + 4u * i) * 1024u);
+  };
+  load_k(start, 0);
+  T8 qf[4];
+  load_q(static_cast<const T*>(a.q) + plane, q, qin, g, qf);
+  if (nkb > 1) load_k(start + KB, 1);
+  int off[4];
+  fragment_offsets(lane, off);
+
+  f32x16 o[2], s[2][2];  // s[j % 2]: the scores of block j
+#pragma unroll
+  for (int d = 0; d < 2; ++d)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[d][r] = 0.f;
+  T8 p[4];  // probabilities of the block before
+  float mrow = -INFINITY, lsum = 0.f;
+  const bool active = row0 + wave * 32 < row1;  // waves past the tile's last row only stage keys
+
+  auto scores = [&](const T* k, f32x16 (&t)[2]) {
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) t[kt][r] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        t[kt] = mfma32(*reinterpret_cast<const T8*>(k + off[ks] + kt * 32 * 64), qf[ks], t[kt]);
+    }
+  };
+  auto weigh = [&](const T* v) {  // O^T += V^T P^T
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int d = 0; d < 2; ++d) o[d] = mfma32(*reinterpret_cast<const T8*>(v + off[c] + d * 32 * KB), p[c], o[d]);
+  };
+  // Block j (P = j % 2): K(j + 1) and V(j - 1) have landed; K(j + 2) and V(j) take the buffers of K(j)
+  // and V(j - 2), whose reads the barrier has ended.
+  // Probabilities of block j against the row's reference max, and this lane's sum of them (of the 16-bit
+  // values that multiply V).
+  constexpr float kScale = 0.125f * 1.4426950408889634f;  // 1/sqrt(64) in the exp2 domain
+  auto probabilities = [&](const f32x16 (&t)[2]) {
+    float rs[2] = {0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        p[c][e] = to_half<T>(__builtin_amdgcn_exp2f(__builtin_fmaf(t[c >> 1][8 * (c & 1) + e], kScale, -mrow)));
+      rs[0] = sum2(__builtin_shufflevector(p[c], p[c], 0, 1), rs[0]);
+      rs[1] = sum2(__builtin_shufflevector(p[c], p[c], 2, 3), rs[1]);
+      rs[0] = sum2(__builtin_shufflevector(p[c], p[c], 4, 5), rs[0]);
+      rs[1] = sum2(__builtin_shufflevector(p[c], p[c], 6, 7), rs[1]);
+    }
+    return rs[0] + rs[1];
+  };
+  auto block_max = [&](const f32x16 (&t)[2]) {
+    float mx = max3_after_mfma(t[0][0], t[0][1], t[0][2]);
+#pragma unroll
+    for (int r = 3; r < 15; r += 2) mx = max3(mx, t[0][r], t[0][r + 1]);
+    mx = max3(mx, t[0][15], t[1][15]);
+#pragma unroll
+    for (int r = 0; r < 14; r += 2) mx = max3(mx, t[1][r], t[1][r + 1]);
+    return half_max(max3(mx, t[1][14], t[1][14])) * kScale;
+  };
+  // Every step runs the scores of the next block; those of the one past the last read the stage's
+  // previous block and are never used, which keeps the step one straight line.
+  auto step = [&](int j, auto parity, auto first_c) {
+    constexpr int P = decltype(parity)::value;
+    constexpr bool first = decltype(first_c)::value;
+    publish_stage<waitcnt_vm(0)>();
+    if (j + 2 < nkb) load_k(start + (j + 2) * KB, P);
+    load_v(start + j * KB, P);
+    if (!active) return;
+    if (j + 1 == nkb) {  // keys past the sequence's end
+      const int left = len - j * KB - 8 * g;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[P][kt][r] = kt * 32 + 16 * (r >> 3) + (r & 7) >= left ? -INFINITY : s[P][kt][r];
+    }
+    if constexpr (first) mrow = block_max(s[P]);
+    else weigh(sv[P ^ 1]);
+    float sum = probabilities(s[P]);
+    scores(sk[P ^ 1], s[P ^ 1]);
+    // The reference stays the first block's max until a lane's 32 probabilities pass 32 x 2^8 (16-bit
+    // values hold 2^15): below that no block needs its maximum.  The sum cannot pass it without a
+    // probability above 2^8, whose row then moves its reference.
+    if (__builtin_amdgcn_ballot_w64(!(sum <= 8192.f))) {
+      const float bmax = block_max(s[P]);
+      const bool grow = bmax > mrow + 8.f;
+      const float alpha = grow ? __builtin_amdgcn_exp2f(mrow - bmax) : 1.f;
+      mrow = grow ? bmax : mrow;
+      lsum *= alpha;
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+      sum = probabilities(s[P]);
+    }
+    lsum += sum;
+  };
+  publish_stage<waitcnt_vm(0)>();
+  if (active) scores(sk[0], s[0]);
+  typedef std::integral_constant<int, 0> Even;
+  typedef std::integral_constant<int, 1> Odd;
+  step(0, Even(), std::true_type());
+  for (int j = 1; j < nkb; j += 2) {
+    step(j, Odd(), std::false_type());
+    if (j + 1 < nkb) step(j + 1, Even(), std::false_type());
+  }
+  publish_stage<waitcnt_vm(0)>();
+  if (active) weigh(sv[(nkb - 1) & 1]);
+
+  if (!qin) return;
+  const float total = half_sum(lsum);
+  const float inv = qvalid ? 1.0f / total : 0.f;
+  T* orow = out + static_cast<size_t>(q) * ld + head * 64;
+#pragma unroll
+  for (int d = 0; d < 2; ++d)
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) {
+      T4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = to_half<T>(qvalid ? o[d][4 * r4 + e] * inv : 0.f);
+      *reinterpret_cast<T4*>(orow + d * 32 + 8 * r4 + 4 * g) = v;
+    }
+}
+
 template <typename T, int NW>
 __global__ __launch_bounds__(64 * NW) void attention_kernel(AttnArgs a) {
   attention_shared<T, NW>(a);
@@ -701,7 +889,10 @@ hipError_t launch_t(const AttnArgs& a, int mode, int waves, hipStream_t stream) 
     case 1: LAYA_LAUNCH((attention_kernel<T, 1>), grid, dim3(64), 0, stream, a); break;
     case 2: LAYA_LAUNCH((attention_kernel<T, 2>), grid, dim3(128), 0, stream, a); break;
     case 4: LAYA_LAUNCH((attention_kernel<T, 4>), grid, dim3(256), 0, stream, a); break;
-    case 8: LAYA_LAUNCH((attention_kernel8<T>), grid, dim3(512), 0, stream, a); break;
+    case 8:
+      if (a.window < 0) LAYA_LAUNCH((attention_ahead_kernel<T>), dim3(a.max_tiles * 2, a.heads), dim3(256), 0, stream, a);
+      else LAYA_LAUNCH((attention_kernel8<T>), grid, dim3(512), 0, stream, a);
+      break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

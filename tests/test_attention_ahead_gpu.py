@@ -1,0 +1,67 @@
+"""Eight-wave shared attention tiles: the one-block-ahead kernel of global layers (its reference max stays
+the first block's until a block's probabilities grow past 2^8) and the per-wave block skipping of local
+layers, against float64.
+
+Tolerance: the 16-bit rounding of probabilities and output, half a unit each (2^-11 / 2^-8), on rows whose
+weights sum to one over |v| <= 5: 2 x 2^-11 x |v| plus the exponential's fp32 error."""
+import ctypes as ct
+
+import numpy as np
+import pytest
+
+from laya_cuda import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def attend(gpu, lengths, growth, window, dtype):
+    import torch as t
+    lib = _lib.load()
+    heads, half = 2, t.float16 if dtype == "f16" else t.bfloat16
+    starts = np.cumsum([0] + [-(-n // 16) * 16 for n in lengths]).astype(np.int32)
+    m = int(starts[-1]) + 16
+    g = t.Generator(device=gpu).manual_seed(m)
+    q, k = (t.randn((heads, m, 64), generator=g, device=gpu) for _ in range(2))
+    vt = t.randn((heads, 64, m), generator=g, device=gpu).to(half)
+    for a, n in zip(starts, lengths):  # later keys score higher (growth > 1) or lower
+        k[:, a:a + n] *= growth ** (t.arange(n, device=gpu) / 64).floor()[None, :, None]
+    q, k = q.to(half), k.to(half)
+    block, most = lib.laya_attention_block(0, 8), m // 16
+    tiles = np.zeros((most, 4), np.int32)
+    ip = ct.POINTER(ct.c_int32)
+    lens = np.asarray(lengths, np.int32)
+    assert lib.laya_attention_tiles(starts.ctypes.data_as(ip), lens.ctypes.data_as(ip), len(lengths), m, block,
+                                    tiles.ctypes.data_as(ip), most) > 0
+    work = t.from_numpy(tiles).to(gpu)
+    out = t.full((m, heads * 64), float("nan"), dtype=half, device=gpu)
+    _lib.check(lib.laya_op_attention(*(ct.c_void_p(x.data_ptr()) for x in (q, k, vt, out, work)), m, heads, most, 0, 8,
+                                     window, _lib.F16 if dtype == "f16" else _lib.BF16,
+                                     ct.c_void_p(t.cuda.current_stream().cuda_stream)))
+    unit = 2.0 ** -11 if dtype == "f16" else 2.0 ** -8
+    real = t.zeros(m, dtype=t.bool, device=gpu)
+    for a, n in zip(starts.tolist(), lengths):
+        real[a:a + n] = True
+        s = t.matmul(q[:, a:a + n].double(), k[:, a:a + n].double().transpose(1, 2).contiguous()) / 8
+        if window >= 0:
+            at = t.arange(n, device=gpu)
+            s = s.masked_fill((at[:, None] - at[None, :]).abs() > window, float("-inf"))
+        v = vt[:, :, a:a + n].double().transpose(1, 2).contiguous()
+        weights = t.softmax(s, -1)
+        want = t.matmul(weights, v).transpose(0, 1).reshape(n, -1)
+        bound = (t.matmul(weights, v.abs()).transpose(0, 1).reshape(n, -1) * 2 + 0.05) * unit
+        assert ((out[a:a + n].double() - want).abs() <= bound).all(), (a, n)
+    assert (out[~real] == 0).all()
+
+
+# One key, tile edges of 64-key blocks and 128-query halves, a lone second half, several tiles.
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("growth", [1.0, 1.6, 0.5])
+@pytest.mark.parametrize("lengths", [[1], [63, 64, 65], [127, 128, 129, 2], [257], [640, 130, 1024]])
+def test_reference_max_follows_growing_scores(gpu, lengths, growth, dtype):
+    attend(gpu, lengths, growth, -1, dtype)
+
+
+@pytest.mark.parametrize("window", [0, 1, 31, 64, 200])
+@pytest.mark.parametrize("lengths", [[1, 63, 65], [160, 161, 300], [1024]])
+def test_local_blocks_skipped_per_wave(gpu, lengths, window):
+    attend(gpu, lengths, 1.0, window, "f16")

@@ -159,7 +159,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, Acc (&acc)[BM /
           take(i, j, vq, value);
           T4 h;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) h[e] = to_half<T>(gelu16(gate[e]) * value[e]);
+          for (int e = 0; e < 4; ++e) h[e] = to_half<T>(gelu16_rational(gate[e]) * value[e]);
           if constexpr (TN % 2 == 0) {
             *reinterpret_cast<T4*>(stg + r * SP + (j & 1) * 16 + c) = h;
           } else {

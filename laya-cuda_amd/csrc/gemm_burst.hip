@@ -250,7 +250,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_burst_kernel(GemmArgs 
       const int n = (f / 16) * 32 + f % 16;
       const f32x2 g = biased2(r, n), v = biased2(r, n + 16);
       *reinterpret_cast<T2*>(out + static_cast<long long>(row) * a.ldo + n0 / 2 + f) =
-          half2(gelu16(g[0]) * v[0], gelu16(g[1]) * v[1]);
+          half2(gelu16_rational(g[0]) * v[0], gelu16_rational(g[1]) * v[1]);
     }
   } else {
     for (int c = tid; c < BM * BN / 2; c += NT) {

@@ -736,7 +736,7 @@ __global__ __launch_bounds__(64 * NW) void attention_split_kernel(AttnArgs a) {
       for (int w = 0; w < NW; ++w) acc += wt[w] * merged[w * 32 * OP + mq * OP + d0 + e + i];
       v[i] = to_half<T>(valid ? acc * inv : 0.f);
     }
-    *reinterpret_cast<T4*>(orow + e) = v;
+    store_through(orow + e, v);
   }
 }
 
@@ -861,7 +861,7 @@ __global__ __launch_bounds__(64 * NW) void attention_pair_kernel(AttnArgs a) {
       for (int k = 0; k < KG; ++k) acc += wt[k] * merged[(mg + QG * k) * 32 * OP + mr * OP + d0 + e + i];
       v[i] = to_half<T>(valid ? acc * inv : 0.f);
     }
-    *reinterpret_cast<T4*>(orow + e) = v;
+    store_through(orow + e, v);
   }
 }
 

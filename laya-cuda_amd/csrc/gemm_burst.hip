@@ -216,7 +216,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_burst_kernel(GemmArgs 
           v0 = v0 + sbias[n];
           v1 = v1 + sbias[n];
         }
-        if (m0 + r < a.M) *reinterpret_cast<T2*>(vt + static_cast<size_t>(dim(n)) * a.M + m0 + r) = half2(v0, v1);
+        if (m0 + r < a.M) store_through(vt + static_cast<size_t>(dim(n)) * a.M + m0 + r, half2(v0, v1));
       }
       return;
     }
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_burst_kernel(GemmArgs 
         const int r = c / (BN / 2), n = (c % (BN / 2)) * 2, row = m0 + r;
         if (row >= a.M) continue;
         const f32x2 v = biased2(r, n);
-        *reinterpret_cast<T2*>(qk + static_cast<size_t>(row) * 64 + dim(n)) = half2(v[0], v[1]);
+        store_through(qk + static_cast<size_t>(row) * 64 + dim(n), half2(v[0], v[1]));
       }
     } else {
 #pragma unroll
@@ -237,8 +237,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_burst_kernel(GemmArgs 
         const f32x2 cs = rcos[i], sn = rsin[i];
         const f32x2 lo = biased2(r, n), hi = biased2(r, n + BN / 2);
         T* const out = qk + static_cast<size_t>(row) * 64 + d;
-        *reinterpret_cast<T2*>(out) = half2(lo[0] * cs[0] - hi[0] * sn[0], lo[1] * cs[1] - hi[1] * sn[1]);
-        *reinterpret_cast<T2*>(out + 32) = half2(hi[0] * cs[0] + lo[0] * sn[0], hi[1] * cs[1] + lo[1] * sn[1]);
+        store_through(out, half2(lo[0] * cs[0] - hi[0] * sn[0], lo[1] * cs[1] - hi[1] * sn[1]));
+        store_through(out + 32, half2(hi[0] * cs[0] + lo[0] * sn[0], hi[1] * cs[1] + lo[1] * sn[1]));
       }
     }
   } else if constexpr (E == Epi::GEGLU) {
@@ -249,8 +249,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_burst_kernel(GemmArgs 
       if (row >= a.M) continue;
       const int n = (f / 16) * 32 + f % 16;
       const f32x2 g = biased2(r, n), v = biased2(r, n + 16);
-      *reinterpret_cast<T2*>(out + static_cast<long long>(row) * a.ldo + n0 / 2 + f) =
-          half2(gelu16_rational(g[0]) * v[0], gelu16_rational(g[1]) * v[1]);
+      store_through(out + static_cast<long long>(row) * a.ldo + n0 / 2 + f,
+                    half2(gelu16_rational(g[0]) * v[0], gelu16_rational(g[1]) * v[1]));
     }
   } else {
     for (int c = tid; c < BM * BN / 2; c += NT) {
@@ -259,10 +259,10 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_burst_kernel(GemmArgs 
       const f32x2 v = biased2(r, n);
       const long long at = static_cast<long long>(row) * a.ldo + n0 + n;
       if constexpr (E == Epi::F32) {
-        *reinterpret_cast<f32x2*>(static_cast<float*>(a.out) + z * a.split_stride + at) = v;
+        store_through(static_cast<float*>(a.out) + z * a.split_stride + at, v);
       } else {
         auto act = [](float x) { return E == Epi::GELU ? gelu16(x) : E == Epi::RELU ? fmaxf(x, 0.f) : x; };
-        *reinterpret_cast<T2*>(static_cast<T*>(a.out) + at) = half2(act(v[0]), act(v[1]));
+        store_through(static_cast<T*>(a.out) + at, half2(act(v[0]), act(v[1])));
       }
     }
   }

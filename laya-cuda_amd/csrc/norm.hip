@@ -14,7 +14,7 @@ namespace {
 template <int D, typename T>
 __global__ __launch_bounds__(256) void embed_norm_kernel(EmbedArgs a) {
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= a.rows) return;
   NormParams<D> np;
   if (a.gamma) np.load(a.gamma, a.beta, lane);
@@ -37,8 +37,8 @@ __global__ __launch_bounds__(256) void embed_norm_kernel(EmbedArgs a) {
     for (int i = 0; i < D / 64; ++i) v[i] = v[i] + t[i];
   }
   if (a.gamma) normalize<D>(v, np, a.eps);
-  if (a.out32) store_row<D>(a.out32 + static_cast<size_t>(row) * D, lane, v);
-  if (a.out16) store_row16<D, T>(static_cast<T*>(a.out16) + static_cast<size_t>(row) * D, lane, v);
+  if (a.out32) store_row_through<D>(a.out32 + static_cast<size_t>(row) * D, lane, v);
+  if (a.out16) store_row16_through<D, T>(static_cast<T*>(a.out16) + static_cast<size_t>(row) * D, lane, v);
 }
 
 // NS: the number of split-K partials when it is known at launch (1..kMaxFixedSplits), so that
@@ -51,7 +51,7 @@ constexpr int kOneWaveRows = 4096;
 template <int D, typename T, int NS>
 __global__ __launch_bounds__(256) void add_norm_kernel(AddNormArgs a) {
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int row = blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (row >= a.rows) return;
   const size_t off = static_cast<size_t>(row) * D;
   NormParams<D> np;
@@ -106,10 +106,10 @@ __global__ __launch_bounds__(256) void add_norm_kernel(AddNormArgs a) {
 #pragma unroll
     for (int i = 0; i < D / 64; ++i) v[i] = v[i] + t[i];
   }
-  if (a.sum_out) store_row<D>(a.sum_out + off, lane, v);
+  if (a.sum_out) store_row_through<D>(a.sum_out + off, lane, v);
   if (a.gamma) normalize<D>(v, np, a.eps);
-  if (a.out32) store_row<D>(a.out32 + off, lane, v);
-  if (a.out16) store_row16<D, T>(static_cast<T*>(a.out16) + off, lane, v);
+  if (a.out32) store_row_through<D>(a.out32 + off, lane, v);
+  if (a.out16) store_row16_through<D, T>(static_cast<T*>(a.out16) + off, lane, v);
 }
 
 template <typename T>

@@ -62,6 +62,34 @@ __device__ __forceinline__ void store_row16(T* dst, int lane, const float (&v)[D
   }
 }
 
+// The same stores written through L2 (see store_through), `dst` wave-uniform.
+template <int D> __device__ __forceinline__ void store_row_through(float* dst, int lane, const float (&v)[D / 64]) {
+  using R = RowMap<D>;
+  if constexpr (R::V == 4) {
+    const __amdgpu_buffer_rsrc_t res = __builtin_amdgcn_make_buffer_rsrc(dst, 0, D * 4, 0x00020000);
+#pragma unroll
+    for (int c = 0; c < R::C; ++c)
+      store_through16(res, R::index(c, lane, 0) * 4, f32x4{v[c * 4], v[c * 4 + 1], v[c * 4 + 2], v[c * 4 + 3]});
+  } else {
+    store_row<D>(dst, lane, v);
+  }
+}
+template <int D, typename T>
+__device__ __forceinline__ void store_row16_through(T* dst, int lane, const float (&v)[D / 64]) {
+  using R = RowMap<D>;
+  if constexpr (R::V == 4) {
+#pragma unroll
+    for (int c = 0; c < R::C; ++c) {
+      typename Vec4<T>::type t;
+      t[0] = to_half<T>(v[c * 4 + 0]); t[1] = to_half<T>(v[c * 4 + 1]);
+      t[2] = to_half<T>(v[c * 4 + 2]); t[3] = to_half<T>(v[c * 4 + 3]);
+      store_through(dst + R::index(c, lane, 0), t);
+    }
+  } else {
+    store_row16<D, T>(dst, lane, v);
+  }
+}
+
 template <int D, typename T>
 __device__ __forceinline__ void load_row16(const T* src, int lane, float (&v)[D / 64]) {
   using R = RowMap<D>;

@@ -6,13 +6,15 @@
 //
 // Workgroup: 4 or 8 waves on a WM x WN grid; each wave owns (BM/WM) x (BN/WN) made of 32x32 MFMA
 // tiles (8 waves put two waves on each SIMD of the CU, so one issues MFMAs while the other waits on
-// LDS or a barrier).  Two main loops share one epilogue:
+// LDS or a barrier).  The main loops share one epilogue:
 //   gemm_kernel       register-staged tiles: 64-deep K slabs staged through registers into two LDS
 //                     buffers, PF slabs of global loads in flight;
 //   gemm_pipe_kernel  an S-stage pipeline of K slabs loaded straight from global memory into LDS,
 //                     LDS fragment reads of the next k-step overlapped with the MFMAs of the current
 //                     one: deep pipelines of small tiles for batch-1 problems, and for batched
-//                     problems large tiles, the 256x256 ones with a ring of half-slab buffers.
+//                     problems large tiles, the 256x256 ones with a ring of half-slab buffers;
+//   gemm_ring16_kernel  the persistent 256x256 ring with 16x16x32 MFMAs, the batched problems' default.
+// Few rows go to gemm_burst.hip.
 // LDS rows hold one slab row with the 16-byte chunk index XOR-swizzled (swz, swz_k below), so the
 // lanes reading one k-chunk of consecutive rows hit distinct banks.
 //
@@ -1054,6 +1056,10 @@ void gemm_ring_persist_kernel(GemmArgs a) {
 //     64 fragment registers instead of 96 leave room for the tile loop without spills;
 //   * the barrier sits two rows into the slab's last k-step, so the LDS reads it waits for are two
 //     rows old.
+// us, against the better of tiles 19, 21, 22 and 26: 65536 x 1024 x 4096 450 -> 428 (1.29 PFLOP/s), 65536
+// x 3072 x 1024 QKV 412 -> 386, 15,088 x 768 x 3,072 79 -> 75, 5,888-row QKV 30 -> 27 and with RoPE 39 ->
+// 34.  Copies without the loads run the first in 353 us, without the MFMAs in 294: what bounds it is
+// their sum under the card's power limit.
 template <typename T, Epi E>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_ring16_kernel(GemmArgs a) {
@@ -1527,7 +1533,7 @@ hipError_t gemm_prepare() {
   return e;
 }
 
-// Measured plans: for the batch-1 GEMM problems of the encoder shapes in gemm_plans.inc (each timed
+// Measured plans of the op-level fp32 products: for the problems in gemm_plans.inc (each timed
 // on an MI355X through the op-level entry points with every tile and split count), the (tile,
 // split-K) launch that timed fastest where it beat the heuristic below by more than 3%.  Keyed by
 // CU count, so another part keeps the heuristic.

@@ -77,7 +77,7 @@ struct GemmTile {
 };
 int gemm_tile_count();
 GemmTile gemm_tile(int id);
-// Packed rows from which a problem counts as batched: the planner costs tiles by their operand
+// Packed rows from which a problem counts as batched: the heuristic costs tiles by their operand
 // bytes per CU, and shape slots keep the out/down projections as 16-bit rows (no split-K).
 constexpr int kBatchedRows = 4096;
 // Chooses a tile and split count for a problem on `cus` compute units: the cost model

@@ -20,6 +20,7 @@
 //     K's LDS rows hold the keys of each 16-key group in the order 0-3, 8-11, 4-7, 12-15, which
 //     leaves each lane the scores of 8 consecutive keys, so V^T's LDS rows keep keys in order.
 #include "kernels.hpp"
+#include "ranges.hpp"
 #include <type_traits>
 
 namespace laya {
@@ -460,8 +461,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
   const bool qin = q < row1, qvalid = qin && q < kend;
   const size_t plane = static_cast<size_t>(head) * a.m * 64;
   // K and V^T through buffer resources of this head's planes: a lane's offset in a block is the same for
-  // every block.  Keys past the end of the slot read zeros (K) or the next head dim's first keys and zeros
-  // past the last one's (V^T): they lie past the end of every sequence, and their probabilities are 0.
+  // every block.  Keys past the end of the slot read zeros or other keys (K) or the next head dim's first
+  // keys and zeros past the last one's (V^T): they lie past the end of every sequence, and their
+  // probabilities are 0.
   const unsigned bytes = static_cast<unsigned>(static_cast<size_t>(a.m) * 128);
   const i32x4 rsK = buffer_resource(static_cast<const T*>(a.k) + plane, bytes);
   const i32x4 rsV = buffer_resource(static_cast<const T*>(a.vt) + plane, bytes);
@@ -479,8 +481,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
   const unsigned ldsV[2] = {lds_address(sv[0]), lds_address(sv[1])};
   auto load_k = [&](int kb, int buf) {
 #pragma unroll
-    for (unsigned i = 0; i < 2; ++i)
-      lds_load16_buffer(rsK, srcK, (static_cast<unsigned>(kb) + 32u * i) * 128u, ldsK[buf] + (wave + 4u * i) * 1024u);
+    for (int i = 0; i < 2; ++i)
+      lds_load16_buffer(rsK, srcK, key_half_offset(kb, i, a.m), ldsK[buf] + (wave + 4u * i) * 1024u);
   };
   auto load_v = [&](int kb, int buf) {
 #pragma unroll

@@ -32,6 +32,7 @@
 //   QKV_ROPE - QKV with rotate-half RoPE applied to Q and K in fp32 before the rounding.
 #include "gemm_burst.hpp"
 #include "kernels.hpp"
+#include "ranges.hpp"
 #include "tiles.hpp"
 
 #include <algorithm>
@@ -1093,12 +1094,14 @@ void gemm_ring16_kernel(GemmArgs a) {
   // gemm_ring_persist_kernel): rows past M are outside the A resource and never stored.
   const int lr = lane / CPR, pch = lane % CPR;
   // Load q of a half is 64 rows further on: the same swizzle, so its distance goes into the scalar
-  // offset (the range check is on the sum) and each operand takes one offset register.
+  // offset and each operand takes one offset register.  In a tile's A rows that distance stays inside
+  // the resource (ring_row_offset), as the range check asks.
   const int row0 = wave * RPI + lr;
   const unsigned chunk = static_cast<unsigned>(pch ^ swz_k<BKS>(row0)) << 3;
   const unsigned srcA = (static_cast<unsigned>(row0) * static_cast<unsigned>(a.lda) + chunk) * 2u;
   const unsigned srcB = (static_cast<unsigned>(row0) * static_cast<unsigned>(a.ldb) + chunk) * 2u;
-  const unsigned stepA = NW * RPI * 2u * static_cast<unsigned>(a.lda), stepB = NW * RPI * 2u * static_cast<unsigned>(a.ldb);
+  static_assert(NW * RPI == 64, "ring_row_offset's rows per load");
+  const unsigned rowA = 2u * static_cast<unsigned>(a.lda), stepB = NW * RPI * 2u * static_cast<unsigned>(a.ldb);
   auto res_a = [&](int m0) {
     return buffer_resource(static_cast<const T*>(a.a) + static_cast<size_t>(m0) * a.lda,
                            static_cast<unsigned>(static_cast<size_t>(a.M - m0) * a.lda * 2));
@@ -1122,6 +1125,7 @@ void gemm_ring16_kernel(GemmArgs a) {
   bool has_next = kLoop && nid < total;
   if (has_next) decode(nid, nm0, nn0);
   i32x4 nrsA = res_a(nm0), nrsB = res_b(nn0);
+  unsigned limA = ring_row_limit(a.M - m0, rowA), nlimA = ring_row_limit(a.M - nm0, rowA);
 
   // Load q of the A (or B) half of stream slab `s` counted from this tile's first slab: this tile's
   // slab s, the next tile's slab s - n, or (last tile) this tile's last slab again, never read.
@@ -1129,7 +1133,7 @@ void gemm_ring16_kernel(GemmArgs a) {
     const bool next = s >= n && has_next;
     const int kt = next ? s - n : min(s, n - 1);
     lds_load16_buffer(isB ? (next ? nrsB : rsB) : (next ? nrsA : rsA), isB ? srcB : srcA,
-                      static_cast<unsigned>(kt) * BKS * 2 + q * (isB ? stepB : stepA),
+                      static_cast<unsigned>(kt) * BKS * 2 + (isB ? q * stepB : ring_row_offset(q, rowA, next ? nlimA : limA)),
                       lds_base + static_cast<unsigned>(buf * HALFB + (wave + NW * q) * RPI * BKS * 2));
   };
 
@@ -1279,12 +1283,14 @@ void gemm_ring16_kernel(GemmArgs a) {
     n0 = nn0;
     rsA = nrsA;
     rsB = nrsB;
+    limA = nlimA;
     nid += G;
     has_next = nid < total;
     if (has_next) {
       decode(nid, nm0, nn0);
       nrsA = res_a(nm0);
       nrsB = res_b(nn0);
+      nlimA = ring_row_limit(a.M - nm0, rowA);
     }
     load_tile_inputs();
 #pragma unroll

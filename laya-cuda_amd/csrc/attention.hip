@@ -461,9 +461,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
   const bool qin = q < row1, qvalid = qin && q < kend;
   const size_t plane = static_cast<size_t>(head) * a.m * 64;
   // K and V^T through buffer resources of this head's planes: a lane's offset in a block is the same for
-  // every block.  Keys past the end of the slot read zeros or other keys (K) or the next head dim's first
-  // keys and zeros past the last one's (V^T): they lie past the end of every sequence, and their
-  // probabilities are 0.
+  // every block but V^T's where the slot ends.  Keys past it lie past the end of every sequence: K reads
+  // zeros or other keys there (masked), V^T its row's last eight keys (finite values of this head dim,
+  // times probabilities that are 0).
   const unsigned bytes = static_cast<unsigned>(static_cast<size_t>(a.m) * 128);
   const i32x4 rsK = buffer_resource(static_cast<const T*>(a.k) + plane, bytes);
   const i32x4 rsV = buffer_resource(static_cast<const T*>(a.vt) + plane, bytes);
@@ -485,9 +485,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
       lds_load16_buffer(rsK, srcK, key_half_offset(kb, i, a.m), ldsK[buf] + (wave + 4u * i) * 1024u);
   };
   auto load_v = [&](int kb, int buf) {
+    const bool inside = kb + KB <= a.m;
+    const unsigned at = inside ? srcV : static_cast<unsigned>(tid >> 3) * row_bytes +
+                                            2u * value_chunk_key(kb, (tid & 7) ^ kvswz(tid >> 3), a.m);
 #pragma unroll
     for (unsigned i = 0; i < 2; ++i)
-      lds_load16_buffer(rsV, srcV, static_cast<unsigned>(kb) * 2u + i * 32u * row_bytes, ldsV[buf] + (wave + 4u * i) * 1024u);
+      lds_load16_buffer(rsV, at, (inside ? static_cast<unsigned>(kb) * 2u : 0u) + i * 32u * row_bytes,
+                        ldsV[buf] + (wave + 4u * i) * 1024u);
   };
   load_k(start, 0);
   T8 qf[4];

@@ -22,4 +22,8 @@ constexpr unsigned key_half_offset(int kb, int half, int m) {
   return static_cast<unsigned>(kb + 32 * half < m ? kb + 32 * half : kb) * 128u;
 }
 
+// Attention, V^T rows of m keys: the first of the eight keys of 16-byte chunk c of the block at kb; chunks
+// past the end take the row's last eight keys, values of the same head dim.
+constexpr int value_chunk_key(int kb, int c, int m) { return kb + 8 * c < m - 8 ? kb + 8 * c : m - 8; }
+
 }  // namespace laya

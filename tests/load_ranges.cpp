@@ -1,6 +1,6 @@
-// Walks the addresses of the ring GEMM's A loads and of the one-block-ahead attention kernel's K
+// Walks the addresses of the ring GEMM's A loads and of the one-block-ahead attention kernel's K and V^T
 // loads (laya-cuda_amd/csrc/ranges.hpp) for operands of many sizes: scalar offsets stay inside the resource,
-// and rows and keys that exist are read from their own place.
+// rows and keys that exist are read from their own place, and V^T chunks never leave their head dim's row.
 #include <cstdio>
 #include <cstdlib>
 #include <initializer_list>
@@ -37,6 +37,11 @@ int main() {
       for (int half = 0; half < 2; ++half) {
         const unsigned soffset = laya::key_half_offset(kb, half, m);
         require(soffset < static_cast<unsigned>(m) * 128u, "scalar offset past the K plane", m, kb, half);
+        for (int c = 0; c < 8; ++c) {
+          const int key = laya::value_chunk_key(kb, c, m);
+          require(key >= 0 && key + 8 <= m, "a V^T chunk leaves its row", m, kb, c);
+          if (kb + 8 * c + 8 <= m) require(key == kb + 8 * c, "a V^T chunk is read elsewhere", m, kb, c);
+        }
         if (kb + 32 * half < m) require(soffset == (kb + 32u * static_cast<unsigned>(half)) * 128u, "a K half is read elsewhere", m, kb, half);
         ++checked;
       }

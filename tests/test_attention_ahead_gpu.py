@@ -65,3 +65,30 @@ def test_reference_max_follows_growing_scores(gpu, lengths, growth, dtype):
 @pytest.mark.parametrize("lengths", [[1, 63, 65], [160, 161, 300], [1024]])
 def test_local_blocks_skipped_per_wave(gpu, lengths, window):
     attend(gpu, lengths, 1.0, window, "f16")
+
+
+def test_keys_past_the_slot_bring_no_other_values(gpu):
+    """The last block of the last sequence reaches past the slot: what stands in for its V^T keys there
+    stays with the head dim's last keys, so another sequence's infinite values, times probabilities of
+    zero, make no NaN of it."""
+    import torch as t
+    lib = _lib.load()
+    lengths, m, heads = [64, 70], 160, 2
+    starts, lens = np.array([0, 64], np.int32), np.array(lengths, np.int32)
+    g = t.Generator(device=gpu).manual_seed(4)
+    q, k = (t.randn((heads, m, 64), generator=g, device=gpu).half() for _ in range(2))
+    vt = t.randn((heads, 64, m), generator=g, device=gpu).half()
+    tiles = np.zeros((10, 4), np.int32)
+    ip = ct.POINTER(ct.c_int32)
+    used = lib.laya_attention_tiles(starts.ctypes.data_as(ip), lens.ctypes.data_as(ip), 2, m,
+                                    lib.laya_attention_block(0, 8), tiles.ctypes.data_as(ip), 10)
+    work = t.from_numpy(tiles[:used].copy()).to(gpu)
+
+    def attention(values):
+        out = t.empty((m, heads * 64), dtype=t.float16, device=gpu)
+        _lib.check(lib.laya_op_attention(*(ct.c_void_p(x.data_ptr()) for x in (q, k, values, out, work)), m, heads, used,
+                                         0, 8, -1, _lib.F16, ct.c_void_p(t.cuda.current_stream().cuda_stream)))
+        return out
+    spoiled = vt.clone()
+    spoiled[:, :, :64] = float("inf")
+    assert t.equal(attention(spoiled)[64:134], attention(vt)[64:134])

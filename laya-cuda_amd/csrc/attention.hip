@@ -898,7 +898,8 @@ hipError_t launch_t(const AttnArgs& a, int mode, int waves, hipStream_t stream) 
     case 2: LAYA_LAUNCH((attention_kernel<T, 2>), grid, dim3(128), 0, stream, a); break;
     case 4: LAYA_LAUNCH((attention_kernel<T, 4>), grid, dim3(256), 0, stream, a); break;
     case 8:
-      if (a.window < 0) LAYA_LAUNCH((attention_ahead_kernel<T>), dim3(a.max_tiles * 2, a.heads), dim3(256), 0, stream, a);
+      // The ahead kernel's buffer resources span a head's m rows of 128 bytes with 32-bit offsets.
+      if (a.window < 0 && a.m < (1 << 25)) LAYA_LAUNCH((attention_ahead_kernel<T>), dim3(a.max_tiles * 2, a.heads), dim3(256), 0, stream, a);
       else LAYA_LAUNCH((attention_kernel8<T>), grid, dim3(512), 0, stream, a);
       break;
     default: return hipErrorInvalidValue;

@@ -92,3 +92,24 @@ def test_keys_past_the_slot_bring_no_other_values(gpu):
     spoiled = vt.clone()
     spoiled[:, :, :64] = float("inf")
     assert t.equal(attention(spoiled)[64:134], attention(vt)[64:134])
+
+
+def test_slots_past_the_resources_range(gpu):
+    """2^25 rows: a head's K plane of 4 GiB no longer fits a buffer resource, so the shared-key kernel with
+    64-bit addresses takes it.  One sequence, at the slot's end."""
+    import torch as t
+    lib = _lib.load()
+    m, n = 1 << 25, 200
+    start = m - 208
+    q, k, vt, out = (t.empty(m * 64, dtype=t.float16, device=gpu) for _ in range(4))
+    g = t.Generator(device=gpu).manual_seed(5)
+    qs, ks, vs = (t.randn((208, 64), generator=g, device=gpu).half() for _ in range(3))
+    q.view(m, 64)[start:], k.view(m, 64)[start:] = qs, ks
+    vt.view(64, m)[:, start:] = vs.t()
+    work = t.tensor([[start, m, start, n]], dtype=t.int32, device=gpu)
+    _lib.check(lib.laya_op_attention(*(ct.c_void_p(x.data_ptr()) for x in (q, k, vt, out, work)), m, 1, 1, 0, 8, -1,
+                                     _lib.F16, ct.c_void_p(t.cuda.current_stream().cuda_stream)))
+    weights = t.softmax(qs[:n].double() @ ks[:n].double().t().contiguous() / 8, -1)
+    want, got = weights @ vs[:n].double(), out.view(m, 64)[start:]
+    assert ((got[:n].double() - want).abs() <= (weights @ vs[:n].double().abs() * 2 + 0.05) * 2.0 ** -11).all()
+    assert (got[n:] == 0).all()

@@ -218,9 +218,17 @@ int laya_op_norm(float* residual, const float* branch, int splits, int64_t part_
  * 4: GeGLU, out[M][N/2] = gelu(gate) * value with w's rows in the resident GeGLU interleave
  * (32-row groups: 16 gate rows, then their 16 value rows).  tile -1 lets the planner choose tile
  * and splits (splits ignored): for 16-bit outputs by its cost model, for fp32 by the measured plan
- * table when it holds the problem, else the heuristic; tile -2 takes the heuristic alone. */
+ * table when it holds the problem, else the heuristic; tile -2 takes the heuristic alone.  A planned
+ * fp32 product without bias writes as many partials as the plan splits K: out must hold that many
+ * times M*N floats.  laya_op_plan tells the number beforehand (at most 8). */
 int laya_op_linear(const void* x, const void* w, const float* bias, void* out, int kind,
                    int dtype16, int M, int N, int K, int splits, int tile, void* stream);
+
+/* The launch that tile -1 (or -2) stands for: *planned_tile and *planned_splits for laya_op_linear of
+ * this kind (biased: with a bias), or for laya_op_qkv with N = 3 width, K = width (kind 5; 6 with RoPE).
+ * Host arithmetic only: needs no device. */
+int laya_op_plan(int kind, int dtype16, int M, int N, int K, int biased, int tile, int* planned_tile,
+                 int* planned_splits);
 
 /* QKV projection with the head-major epilogue that replaces `layout` (kernels.cu:68-82):
  * q, k [heads][M][64], vt [heads][64][M].  With rope_cos non-NULL, Q and K are rotated (rotate-half

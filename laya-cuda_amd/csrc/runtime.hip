@@ -1375,21 +1375,40 @@ int laya_op_norm(float* residual, const float* branch, int splits, int64_t part_
   });
 }
 
+// Epilogue of an op-level GEMM kind: 0-4 laya_op_linear's, 5 laya_op_qkv, 6 laya_op_qkv with RoPE.
+static Epi op_epilogue(int kind) {
+  constexpr Epi kinds[] = {Epi::F32, Epi::HALF, Epi::GELU, Epi::RELU, Epi::GEGLU, Epi::QKV, Epi::QKV};
+  return kinds[kind];
+}
+// The planner's launch for an op-level GEMM (tile -1, or -2: the heuristic alone).
+static void plan_op(int kind, int dtype16, int M, int N, int K, bool biased, int* tile, int* splits) {
+  // fp32 plans: the caller sums the split partials, so their number is the table's and heuristic's.
+  const bool planned = *tile == -1;
+  gemm_plan(M, N, K, op_epilogue(kind), half_type(dtype16), 256, tile, splits, kind == 6, planned, planned && kind != 0);
+  if (biased || kind >= 5) *splits = 1;
+}
+
+int laya_op_plan(int kind, int dtype16, int M, int N, int K, int biased, int tile, int* planned_tile,
+                 int* planned_splits) {
+  return guarded(nullptr, [&] {
+    LAYA_REQUIRE(kind >= 0 && kind <= 6, "kind must be 0-4 (laya_op_linear), 5 (laya_op_qkv) or 6 (with RoPE)");
+    LAYA_REQUIRE(tile == -1 || tile == -2, "tile must be -1 (the planner) or -2 (its heuristic)");
+    LAYA_REQUIRE(M > 0 && N > 0 && K > 0 && planned_tile && planned_splits, "positive sizes and both outputs");
+    int splits = 1;
+    plan_op(kind, dtype16, M, N, K, biased != 0, &tile, &splits);
+    *planned_tile = tile;
+    *planned_splits = splits;
+  });
+}
+
 int laya_op_linear(const void* x, const void* w, const float* bias, void* out, int kind, int dtype16, int M, int N,
                    int K, int splits, int tile, void* stream) {
   return guarded(nullptr, [&] {
     prepare_device();
     LAYA_REQUIRE(kind >= 0 && kind <= 4,
                  "kind must be 0 (fp32), 1 (16-bit), 2 (16-bit GELU), 3 (16-bit ReLU) or 4 (16-bit GeGLU)");
-    const Epi epi = kind == 0 ? Epi::F32 : kind == 1 ? Epi::HALF : kind == 2 ? Epi::GELU : kind == 3 ? Epi::RELU
-                                                                                                    : Epi::GEGLU;
-    int cus = 256;
-    if (tile < 0) {
-      // fp32 plans: the caller sums the split partials, so their number is the table's and heuristic's.
-      gemm_plan(M, N, K, epi, half_type(dtype16), cus, &tile, &splits, false, tile == -1,
-                tile == -1 && epi != Epi::F32);
-      if (bias) splits = 1;
-    }
+    const Epi epi = op_epilogue(kind);
+    if (tile < 0) plan_op(kind, dtype16, M, N, K, bias != nullptr, &tile, &splits);
     LAYA_REQUIRE(tile < gemm_tile_count(), "bad tile id");
     LAYA_REQUIRE(K % 64 == 0 && N % gemm_tile(tile).bn == 0, "K must be a multiple of 64 and N of the tile width");
     GemmArgs g{};
@@ -1408,7 +1427,7 @@ int laya_op_qkv(const void* x, const void* w, const float* bias, void* q, void* 
     int splits = 1;
     const bool rope = rope_cos != nullptr;
     LAYA_REQUIRE(!rope || (rope_sin && positions), "RoPE needs cos, sin and positions");
-    if (tile < 0) gemm_plan(M, 3 * width, width, Epi::QKV, half_type(dtype16), 256, &tile, &splits, rope, tile == -1, tile == -1);
+    if (tile < 0) plan_op(rope ? 6 : 5, dtype16, M, 3 * width, width, false, &tile, &splits);
     LAYA_REQUIRE(tile < gemm_tile_count(), "bad tile id");
     LAYA_REQUIRE(width % 64 == 0 && (3 * width) % gemm_tile(tile).bn == 0, "width does not fit the tile");
     LAYA_REQUIRE(M % 8 == 0, "rows must be a multiple of 8 (V^T is stored in runs of 8 tokens)");

@@ -1559,34 +1559,52 @@ namespace {
 
 // Plans by cost: a launch's time follows a + s L nk + r (R - 1) + o MB, where L is the most tiles a CU
 // gets, nk its 64-deep slabs per tile, R the rounds of workgroups (two per CU where LDS allows) and MB
-// the output's megabytes.  The constants are fits to graph replays over weights that are cold in
-// every cache: 14 projections of widths 768 and 1,024 at 12 row counts of 16-512, and 16 at 18 row
-// counts of 640-24,576 (6-12% rms).  Up to 512 rows the choice they make is 2% slower on average than
-// the best tile measured, above 1%, where the plan table with the larger-tile heuristic it
-// replaced was 32% and 13% slower (us: 96-row QKV 6.6 -> 4.7, with RoPE 9.9 -> 4.9; 1,008-row GELU
-// up 18.1 -> 13.1, GeGLU up 14.1 -> 10.0, 768 x 768 with fp32 output 9.2 -> 6.0).  An fp32 split costs
-// its consumer another partial to read (0.12 us per 512 rows), and splits stop where the partials
-// would pass 16 MB.
+// the output's megabytes, with an own rate for fp32 output (o32) and an addition for RoPE (p).  Where the
+// tile count is no multiple of the 8 XCDs the tiles are walked row by row across them, and each of the
+// tile columns fetches A into another L2: q per megabyte of A, at most 8 times.
+// Up to 512 rows the constants are fits to graph replays over weights that are cold in every cache (14
+// projections of widths 768 and 1,024 at 12 row counts).  Above, they are fits to the stage times of each
+// tile inside whole forwards of three encoders at 21 to 31 row classes and to replays of 700 problems
+// of random kind, depth and row count (tune_gemm_costs.py and its data): replays alone rank the tiles
+// otherwise than a forward does (constants fitted to them chose 128x256 tiles for down projections that
+// run 17% slower in it).  How far the choice is from the best tile measured, on average: 0.5% on 117
+// other replayed problems up to 512 rows; above, 0.9% on row classes and 0.7% on problems that were left out
+// of a fit made for that check, worst 14%.  Constants without q, o32 and p, fitted to replays at 18 row
+// counts, were 1.6% and 4.2% off, worst 24% and 35% (7,825 x 768 x 1,152 32.4 us against 24.4 by the
+// plan table and heuristic before them, 25.7 now; 15,104 x 768 x 768 in a forward 29.9 against 24.2 now), and
+// the table and heuristic 20-27% (us: 96-row QKV 6.6 -> 4.7, with RoPE 9.9 -> 4.9; 1,008-row GeGLU up
+// 14.1 -> 9.1).
+// An fp32 split costs its consumer another partial to read (0.12 us per 512 rows), and splits stop where
+// the partials would pass 16 MB.
 constexpr int kFewRows = 512;
 constexpr int kCostDepth = 512;  // shallower products (widths below 512) were not measured
 struct TileCost {
   int tile, per_cu;
-  float a, s, r, o;
+  float a, s, r, o, o32, q, p;
   int max_slabs = 1 << 30;
 };
 constexpr TileCost kFewRowCosts[] = {
-    {27, 2, 2.85f, 0.114f, 1.12f, 0.195f}, {28, 1, 3.06f, 0.144f, 1.99f, 0.134f}, {29, 1, 3.01f, 0.182f, 2.07f, 0.140f},
-    {30, 1, 2.98f, 0.202f, 1.89f, 0.204f}, {31, 1, 2.91f, 0.263f, 1.58f, 0.216f}, {32, 1, 3.35f, 0.237f, 2.04f, 0.231f},
-    {33, 1, 3.16f, 0.344f, 1.61f, 0.252f}, {34, 1, 3.08f, 0.400f, 1.47f, 0.206f}, {14, 1, 2.94f, 0.254f, 1.42f, 0.267f},
-    {23, 1, 2.83f, 0.332f, 1.21f, 0.281f}, {24, 1, 2.69f, 0.392f, 1.10f, 0.262f},
+    {27, 2, 2.85f, 0.114f, 1.12f, 0.195f, 0.195f}, {28, 1, 3.06f, 0.144f, 1.99f, 0.134f, 0.134f},
+    {29, 1, 3.01f, 0.182f, 2.07f, 0.140f, 0.140f}, {30, 1, 2.98f, 0.202f, 1.89f, 0.204f, 0.204f},
+    {31, 1, 2.91f, 0.263f, 1.58f, 0.216f, 0.216f}, {32, 1, 3.35f, 0.237f, 2.04f, 0.231f, 0.231f},
+    {33, 1, 3.16f, 0.344f, 1.61f, 0.252f, 0.252f}, {34, 1, 3.08f, 0.400f, 1.47f, 0.206f, 0.206f},
+    {14, 1, 2.94f, 0.254f, 1.42f, 0.267f, 0.267f}, {23, 1, 2.83f, 0.332f, 1.21f, 0.281f, 0.281f},
+    {24, 1, 2.69f, 0.392f, 1.10f, 0.262f, 0.262f},
 };
 // Tile 21's two-stage pipeline falls behind with depth (15,088 x 768: 26.5 against the ring's 24.2 us at
-// K = 768 but 92 against 76 at 3,072), so it is kept to the depths its constants were fitted on.
+// K = 768 but 92 against 76 at 3,072), so it is kept to 16 slabs.
 constexpr TileCost kCosts[] = {
-    {14, 1, 3.92f, 0.198f, 2.17f, 0.048f}, {31, 1, 3.45f, 0.252f, 2.08f, 0.019f}, {34, 1, 3.76f, 0.389f, 2.30f, 0.074f},
-    {23, 1, 3.70f, 0.274f, 2.00f, 0.127f}, {24, 1, 3.83f, 0.275f, 2.02f, 0.109f}, {16, 1, 4.20f, 0.271f, 1.88f, 0.386f},
-    {25, 1, 4.02f, 0.394f, 3.31f, 0.132f}, {18, 1, 4.47f, 0.401f, 3.59f, 0.114f}, {9, 1, 4.32f, 0.902f, 1.80f, 0.321f},
-    {8, 1, 4.38f, 0.907f, 2.10f, 0.288f},  {21, 1, 6.58f, 0.962f, 4.89f, 0.257f, 16}, {35, 1, 6.28f, 1.026f, 3.28f, 0.380f},
+    {14, 1, 3.108f, 0.204f, 0.919f, 0.644f, 0.320f, 0.027f, 0.f},
+    {31, 1, 2.083f, 0.257f, 0.716f, 0.785f, 0.336f, 0.f, 0.164f},
+    {34, 1, 2.110f, 0.430f, 1.189f, 0.486f, 0.178f, 0.f, 0.055f},
+    {23, 1, 2.924f, 0.309f, 0.712f, 0.443f, 0.247f, 0.015f, 0.f},
+    {24, 1, 2.879f, 0.311f, 0.604f, 0.482f, 0.251f, 0.013f, 0.f},
+    {25, 1, 2.776f, 0.450f, 0.159f, 0.504f, 0.247f, 0.015f, 0.113f},
+    {18, 1, 3.346f, 0.452f, 0.662f, 0.430f, 0.220f, 0.016f, 0.145f},
+    {9, 1, 3.938f, 0.972f, 0.415f, 0.354f, 0.155f, 0.013f, 0.089f},
+    {8, 1, 3.871f, 0.954f, 0.959f, 0.323f, 0.145f, 0.017f, 0.097f},
+    {21, 1, 5.205f, 1.065f, 2.073f, 0.347f, 0.121f, 0.013f, 0.f, 16},
+    {35, 1, 6.335f, 1.098f, 4.732f, 0.245f, 0.f, 0.002f, 0.299f},
 };
 
 template <size_t C>
@@ -1605,8 +1623,10 @@ bool cost_plan(const TileCost (&costs)[C], int M, int N, int K, Epi epi, int cus
       if (z > 1 && (nk < 2 * z || static_cast<long long>(M) * N * 4 * z > (16LL << 20))) break;
       const long long work = tiles * z, rounds = (work + cus * c.per_cu - 1) / (cus * c.per_cu);
       const float mb = static_cast<float>(M) * N * (epi == Epi::F32 ? 4 * z : 2) * 1e-6f;
+      const float per_mb = epi == Epi::F32 ? c.o32 : rope ? c.o + c.p : c.o;
+      const float a_mb = work % 8 ? static_cast<float>(std::min(8, N / d.bn)) * M * K * 2e-6f : 0.f;
       const float t = c.a + c.s * static_cast<float>((work + cus - 1) / cus * ((nk + z - 1) / z)) +
-                      c.r * static_cast<float>(rounds - 1) + c.o * mb +
+                      c.r * static_cast<float>(rounds - 1) + per_mb * mb + c.q * a_mb +
                       (epi == Epi::F32 ? 0.12f * z * static_cast<float>(std::max(M, 512)) / 512.f : 0.f);
       if (best < 0.f || t < best) {
         best = t;

@@ -1,6 +1,9 @@
 """laya_op_plan: the tile and split count that laya_op_linear's and laya_op_qkv's planned launches (tile -1)
 take, known before the call (no GPU but for the test that a planned fp32 product writes exactly that many partials)."""
 import ctypes as ct
+import gzip
+import json
+from pathlib import Path
 
 import pytest
 
@@ -33,6 +36,24 @@ def test_bad_plan_requests_are_refused():
                  (1, _lib.F16, 16, 64, 64, 0, 3)]:
         assert lib.laya_op_plan(*args, ct.byref(t), ct.byref(t)) == _lib.EINVAL
     assert lib.laya_op_plan(1, _lib.F16, 16, 64, 64, 0, -1, None, None) == _lib.EINVAL
+
+
+DATA = Path(__file__).resolve().parents[1] / "laya-cuda_amd" / "csrc" / "gemm_cost_data.json.gz"
+
+
+@pytest.mark.parametrize("where,mean,most", [("forward", 1.01, 1.14), ("held_out", 1.01, 1.15), ("isolated", 1.01, 1.25)])
+def test_planned_tiles_are_near_the_best_measured(where, mean, most):
+    """The planner's choice for 16-bit products of more than 512 rows against the times that its constants come
+    from (measured inside forwards and as isolated launches).  The bounds are what the constants reach:
+    mean 1.008, 1.007 and 1.009, largest 1.134, 1.145 and 1.239."""
+    kinds = {"half": 1, "gelu": 2, "relu": 3, "geglu": 4, "qkv": 5, "rope": 6}
+    ratios = []
+    for kind, M, N, K, timed in json.loads(gzip.decompress(DATA.read_bytes()))[where]:
+        if M > 512 and kind in kinds:
+            us = {tile: t for tile, _, t, _ in timed}
+            ratios.append(us[plan(kinds[kind], M, N, K)[0]] / min(us.values()))
+    assert len(ratios) > 100
+    assert sum(ratios) / len(ratios) <= mean and max(ratios) <= most
 
 
 @pytest.mark.gpu

@@ -314,7 +314,8 @@ __device__ __forceinline__ void load_q(const T* Q, int q, bool qin, int g, typen
 // Large batches: a workgroup of NW waves owns 32*NW queries of one sequence and one head; every
 // K/V block is staged once in LDS (double-buffered, the next block's global loads in flight during
 // the current block's MFMAs) and shared by all NW waves.
-template <typename T, int NW>
+// kGlobal: the caller has no window (the code for local layers is left out).
+template <typename T, int NW, bool kGlobal = false>
 __device__ __forceinline__ void attention_shared(const AttnArgs& a) {
   typedef typename Vec8<T>::type T8;
   typedef typename Vec4<T>::type T4;
@@ -373,7 +374,7 @@ __device__ __forceinline__ void attention_shared(const AttnArgs& a) {
 
   // Keys this tile can see: the whole sequence, or on local layers the window around its rows
   // (first block 16-aligned, so the 16-byte V^T loads stay aligned); this lane's query sees [qlo, qhi).
-  const bool local = a.window >= 0;
+  const bool local = !kGlobal && a.window >= 0;
   const int klo = local ? max(start, (row0 - a.window) & ~15) : start;
   const int khi = local ? min(kend, row1 + a.window) : kend;
   const int nkb = (khi - klo + KB - 1) / KB;
@@ -400,8 +401,9 @@ __device__ __forceinline__ void attention_shared(const AttnArgs& a) {
     constexpr int cur = decltype(cur_c)::value;
     const int kb = klo + j * KB;
     if (j + 1 < nkb) kv_load_direct<T, NT>(K, Vt, a.m, kb + KB, ldsK[cur ^ 1], ldsV[cur ^ 1], tid, uwave);
-    if (active && kb < whi && kb + KB > wlo)
-      attend_block<T>(cur ? frag1 : frag0, qf, o, mrow, lsum, kb, kb < all_lo || kb + KB > all_hi, qlo, qhi, lane);
+    if (active && (kGlobal || (kb < whi && kb + KB > wlo)))
+      attend_block<T>(cur ? frag1 : frag0, qf, o, mrow, lsum, kb, (!kGlobal && kb < all_lo) || kb + KB > all_hi, qlo, qhi,
+                      lane);
     publish_stage<waitcnt_vm(0)>();
   };
   for (int j = 0; j < nkb; j += 2) {
@@ -485,13 +487,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
       lds_load16_buffer(rsK, srcK, key_half_offset(kb, i, a.m), ldsK[buf] + (wave + 4u * i) * 1024u);
   };
   auto load_v = [&](int kb, int buf) {
-    const bool inside = kb + KB <= a.m;
-    const unsigned at = inside ? srcV : static_cast<unsigned>(tid >> 3) * row_bytes +
-                                            2u * value_chunk_key(kb, (tid & 7) ^ kvswz(tid >> 3), a.m);
+    if (kb + KB <= a.m) {
 #pragma unroll
-    for (unsigned i = 0; i < 2; ++i)
-      lds_load16_buffer(rsV, at, (inside ? static_cast<unsigned>(kb) * 2u : 0u) + i * 32u * row_bytes,
-                        ldsV[buf] + (wave + 4u * i) * 1024u);
+      for (unsigned i = 0; i < 2; ++i)
+        lds_load16_buffer(rsV, srcV, static_cast<unsigned>(kb) * 2u + i * 32u * row_bytes, ldsV[buf] + (wave + 4u * i) * 1024u);
+    } else {  // a branch, so that only the slot's last block pays for the addresses
+      const unsigned at = static_cast<unsigned>(tid >> 3) * row_bytes +
+                          2u * value_chunk_key(kb, (tid & 7) ^ kvswz(tid >> 3), a.m);
+#pragma unroll
+      for (unsigned i = 0; i < 2; ++i)
+        lds_load16_buffer(rsV, at, i * 32u * row_bytes, ldsV[buf] + (wave + 4u * i) * 1024u);
+    }
   };
   load_k(start, 0);
   T8 qf[4];
@@ -622,9 +628,9 @@ __global__ __launch_bounds__(64 * NW) void attention_kernel(AttnArgs a) {
   attention_shared<T, NW>(a);
 }
 // Eight waves: capped at 128 VGPRs so that two 512-thread workgroups share a CU.
-template <typename T>
+template <typename T, bool kGlobal>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void attention_kernel8(AttnArgs a) {
-  attention_shared<T, 8>(a);
+  attention_shared<T, 8, kGlobal>(a);
 }
 
 // Small batches (few query tiles): a workgroup owns 32 queries of one sequence and one head, and
@@ -873,6 +879,17 @@ __global__ __launch_bounds__(64 * NW) void attention_pair_kernel(AttnArgs a) {
   }
 }
 
+// Whether a tile list known to the host holds so few rows per 256-row tile that the ahead kernel loses: of the
+// two workgroups it starts per tile the second has nothing to do where a sequence ends within 128 rows,
+// and that costs more than the overlap gains.  us, shared keys against one block ahead, 12 heads: 256 x
+// 64 tokens 25.0 and 32.6, 128 x 128 tokens 23.7 and 31.4, 102 x 160 28.9 and 31.2, 53 x 300 (152 rows per tile)
+// 40.4 and 38.2, 40 of 100-512 (190) 35.9 and 33.1, 64 x 256 27.9 and 27.5, 6 x 1,024 38.8 and 31.9.  A slot's
+// list is filled per request, after its kernels are chosen, and keeps the ahead kernel.
+constexpr int kAheadTileRows = 168;
+bool short_tiles(const AttnArgs& a) {
+  return !a.n_tiles && a.m < static_cast<long long>(kAheadTileRows) * a.max_tiles;
+}
+
 template <typename T>
 hipError_t launch_t(const AttnArgs& a, int mode, int waves, hipStream_t stream) {
   const dim3 grid(a.max_tiles, a.heads);
@@ -899,8 +916,10 @@ hipError_t launch_t(const AttnArgs& a, int mode, int waves, hipStream_t stream) 
     case 4: LAYA_LAUNCH((attention_kernel<T, 4>), grid, dim3(256), 0, stream, a); break;
     case 8:
       // The ahead kernel's buffer resources span a head's m rows of 128 bytes with 32-bit offsets.
-      if (a.window < 0 && a.m < (1 << 25)) LAYA_LAUNCH((attention_ahead_kernel<T>), dim3(a.max_tiles * 2, a.heads), dim3(256), 0, stream, a);
-      else LAYA_LAUNCH((attention_kernel8<T>), grid, dim3(512), 0, stream, a);
+      if (a.window < 0 && a.m < (1 << 25) && !short_tiles(a))
+        LAYA_LAUNCH((attention_ahead_kernel<T>), dim3(a.max_tiles * 2, a.heads), dim3(256), 0, stream, a);
+      else if (a.window < 0) LAYA_LAUNCH((attention_kernel8<T, true>), grid, dim3(512), 0, stream, a);
+      else LAYA_LAUNCH((attention_kernel8<T, false>), grid, dim3(512), 0, stream, a);
       break;
     default: return hipErrorInvalidValue;
   }

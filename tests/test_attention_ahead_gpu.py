@@ -1,6 +1,6 @@
 """Eight-wave shared attention tiles: the one-block-ahead kernel of global layers (its reference max stays
-the first block's until a block's probabilities grow past 2^8) and the per-wave block skipping of local
-layers, against float64.
+the first block's until a block's probabilities grow past 2^8), the shared-key kernel that serves short
+sequences, and the per-wave block skipping of local layers, against float64.
 
 Tolerance: the 16-bit rounding of probabilities and output, half a unit each (2^-11 / 2^-8), on rows whose
 weights sum to one over |v| <= 5: 2 x 2^-11 x |v| plus the exponential's fp32 error."""
@@ -14,7 +14,7 @@ from laya_cuda import _lib
 pytestmark = pytest.mark.gpu
 
 
-def attend(gpu, lengths, growth, window, dtype):
+def attend(gpu, lengths, growth, window, dtype, ahead=False):
     import torch as t
     lib = _lib.load()
     heads, half = 2, t.float16 if dtype == "f16" else t.bfloat16
@@ -24,15 +24,16 @@ def attend(gpu, lengths, growth, window, dtype):
     q, k = (t.randn((heads, m, 64), generator=g, device=gpu) for _ in range(2))
     vt = t.randn((heads, 64, m), generator=g, device=gpu).to(half)
     for a, n in zip(starts, lengths):  # later keys score higher (growth > 1) or lower
-        k[:, a:a + n] *= growth ** (t.arange(n, device=gpu) / 64).floor()[None, :, None]
+        k[:, a:a + n] *= growth ** (t.arange(n, device=gpu) / 64).floor().clamp(max=15)[None, :, None]
     q, k = q.to(half), k.to(half)
     block, most = lib.laya_attention_block(0, 8), m // 16
     tiles = np.zeros((most, 4), np.int32)
     ip = ct.POINTER(ct.c_int32)
     lens = np.asarray(lengths, np.int32)
-    assert lib.laya_attention_tiles(starts.ctypes.data_as(ip), lens.ctypes.data_as(ip), len(lengths), m, block,
-                                    tiles.ctypes.data_as(ip), most) > 0
-    work = t.from_numpy(tiles).to(gpu)
+    most = lib.laya_attention_tiles(starts.ctypes.data_as(ip), lens.ctypes.data_as(ip), len(lengths), m, block,
+                                    tiles.ctypes.data_as(ip), most)
+    assert most > 0 and (window >= 0 or (m >= 168 * most) == ahead)
+    work = t.from_numpy(tiles[:most].copy()).to(gpu)
     out = t.full((m, heads * 64), float("nan"), dtype=half, device=gpu)
     _lib.check(lib.laya_op_attention(*(ct.c_void_p(x.data_ptr()) for x in (q, k, vt, out, work)), m, heads, most, 0, 8,
                                      window, _lib.F16 if dtype == "f16" else _lib.BF16,
@@ -53,12 +54,20 @@ def attend(gpu, lengths, growth, window, dtype):
     assert (out[~real] == 0).all()
 
 
-# One key, tile edges of 64-key blocks and 128-query halves, a lone second half, several tiles.
+# One key, tile edges of 64-key blocks and 128-query halves, a lone second half, several tiles; each among
+# longer sequences, whose tiles take the list past the rows per tile from which the ahead kernel serves it.
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("growth", [1.0, 1.6, 0.5])
-@pytest.mark.parametrize("lengths", [[1], [63, 64, 65], [127, 128, 129, 2], [257], [640, 130, 1024]])
+@pytest.mark.parametrize("lengths", [[1, 1024], [63, 64, 65, 2048], [127, 128, 129, 2, 3072], [257, 1024], [640, 130, 1024]])
 def test_reference_max_follows_growing_scores(gpu, lengths, growth, dtype):
-    attend(gpu, lengths, growth, -1, dtype)
+    attend(gpu, lengths, growth, -1, dtype, ahead=True)
+
+
+# Short sequences keep the shared-key kernel.
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("lengths", [[1], [63, 64, 65], [127, 128, 129, 2], [257]])
+def test_short_global_sequences(gpu, lengths, dtype):
+    attend(gpu, lengths, 1.6, -1, dtype)
 
 
 @pytest.mark.parametrize("window", [0, 1, 31, 64, 200])
@@ -73,7 +82,7 @@ def test_keys_past_the_slot_bring_no_other_values(gpu):
     zero, make no NaN of it."""
     import torch as t
     lib = _lib.load()
-    lengths, m, heads = [64, 70], 160, 2
+    lengths, m, heads = [64, 1030], 1104, 2
     starts, lens = np.array([0, 64], np.int32), np.array(lengths, np.int32)
     g = t.Generator(device=gpu).manual_seed(4)
     q, k = (t.randn((heads, m, 64), generator=g, device=gpu).half() for _ in range(2))
@@ -91,7 +100,8 @@ def test_keys_past_the_slot_bring_no_other_values(gpu):
         return out
     spoiled = vt.clone()
     spoiled[:, :, :64] = float("inf")
-    assert t.equal(attention(spoiled)[64:134], attention(vt)[64:134])
+    assert m >= 168 * used  # the ahead kernel
+    assert t.equal(attention(spoiled)[64:1094], attention(vt)[64:1094])
 
 
 def test_slots_past_the_resources_range(gpu):

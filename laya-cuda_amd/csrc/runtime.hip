@@ -431,6 +431,19 @@ size_t carve_slot(const Engine& E, Slot* s, char* base) {
   return at;
 }
 
+// Plans a slot and returns its arena size.  Where laya_predict_static's scratch would hold the arena with
+// fewer split-K partials than the cost model likes, both entry points take the plan that fits: their sums
+// are associated alike whichever of them runs a shape.
+size_t plan_arena(const Engine& E, Slot* s, int m, int b, int k) {
+  for (int max_splits = 8; max_splits; max_splits /= 2) {
+    plan_slot(E, s, m, b, k, max_splits);
+    const size_t bytes = carve_slot(E, s, nullptr);
+    if (bytes <= kScratchBytes) return bytes;
+  }
+  plan_slot(E, s, m, b, k);  // past the scratch either way
+  return carve_slot(E, s, nullptr);
+}
+
 // Host side of Slot.fill's contract: validate the caller's block, then derive the attention tile
 // list and the compact head-row list into the same staging buffer (packing.cpp).
 void derive_inputs(const Engine& E, Slot& s) {
@@ -721,8 +734,7 @@ void forward(Engine& E, Slot& s, int marked = -1, hipEvent_t* marks = nullptr) {
 Slot* create_slot(Engine& E, int m, int b, int k) {
   Slot* s = new Slot();
   try {
-    plan_slot(E, s, m, b, k);
-    const size_t total = carve_slot(E, s, nullptr);
+    const size_t total = plan_arena(E, s, m, b, k);
     LAYA_HIP(hipMalloc(&s->arena, total));
     s->bytes = total;
     E.slot_bytes += total;
@@ -1162,12 +1174,7 @@ int laya_predict_static(void* handle, const int32_t* host_packed, const LayaShap
     LAYA_REQUIRE(m > 0 && m % 16 == 0 && m <= (1 << 22) && b > 0 && b <= (1 << 16) && k > 0 && k <= (1 << 12),
                  "invalid shape class");
     Slot s;  // plans and views into the scratch; owns nothing
-    plan_slot(*E, &s, m, b, k);
-    size_t need = carve_slot(*E, &s, nullptr);
-    if (need > kScratchBytes) {  // without the cost model's split-K partials it may still fit
-      plan_slot(*E, &s, m, b, k, 1);
-      need = carve_slot(*E, &s, nullptr);
-    }
+    const size_t need = plan_arena(*E, &s, m, b, k);
     LAYA_REQUIRE(need <= kScratchBytes,
                  "shape class (" + std::to_string(m) + ", " + std::to_string(b) + ", " + std::to_string(k) +
                      ") needs " + std::to_string(need) + " bytes of device scratch; laya_predict_static holds " +

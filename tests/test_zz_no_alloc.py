@@ -1,8 +1,9 @@
 """laya_predict_static (the entry point that allocates nothing) against laya_predict, through the C
 ABI: bit-identical logits and acts on two calls in a row, the second with a smaller request, both
 on the same engine and the same device scratch; a shape class whose arena exceeds the scratch is
-refused.  The kernels and launch plans are those of laya_predict's forward, so the outputs must
-match it bit for bit (its graph replay equals its eager pass bit for bit).
+refused.  The kernels and launch plans are those of laya_predict's forward (also where the scratch holds
+the arena only with fewer split-K partials), so the outputs must match it bit for bit (its graph replay
+equals its eager pass bit for bit).
 """
 import ctypes as ct
 
@@ -79,5 +80,28 @@ def test_static_entry_point_matches_predict_for_modernbert(gpu):
             np.testing.assert_array_equal(logits, want_logits)
             np.testing.assert_array_equal(acts, want_acts)
             assert np.isfinite(logits).all() and metrics.gpu_ms > 0
+    finally:
+        rt.close()
+
+
+def test_static_entry_point_matches_predict_where_the_partials_fill_the_scratch(gpu):
+    """2,048 rows of a 1,024-wide encoder with 16 questions of up to 16 options: with the down projection's two
+    split-K partials the arena passes the scratch, without them it fits.  Both entry points take that plan."""
+    spec = synthetic.adapter(None, layers=2, width=1024, heads=16, intermediate=4096, vocab=2000, positions=1024,
+                             max_len=1024, mfma_dtype="float16")
+    rt = Runtime(spec, 0, 2, weights=synthetic.weights(spec, seed=3, random_norms=True))
+    try:
+        rng = np.random.default_rng(8)
+        sequences = [rng.integers(5, 2000, 1024, dtype=np.int32) for _ in range(2)]
+        questions = [(i % 2, [1 + i, 40 + i, 1000], 0) for i in range(16)]
+        key = (2048, 16, 16)
+        rc, logits, acts, _ = static_predict(rt, sequences, questions, key=key)
+        assert rc == _lib.OK, _lib.error(rt._handle)
+        before = rt.pool.used_bytes()
+        want_logits, want_acts, _ = rt.predict_sequences(sequences, questions, key=key)
+        np.testing.assert_array_equal(logits, want_logits)
+        np.testing.assert_array_equal(acts, want_acts)
+        arena, partial = rt.pool.used_bytes() - before, 2048 * 1024 * 4
+        assert arena <= 64 << 20 < arena + partial
     finally:
         rt.close()

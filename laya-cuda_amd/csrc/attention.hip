@@ -432,10 +432,11 @@ __device__ __forceinline__ void attention_shared(const AttnArgs& a) {
 // each other, and the barrier of every block lines the waves of a SIMD up in the same phase: 64 x
 // 1,024 tokens ran at their sum.  Here, while the softmax of block j runs, the same wave's matrix
 // instructions are the scores of block j + 1 and the products of block j - 1 with V, which do not
-// depend on it, and no block needs its maximum first (below).  64 x 1,024 tokens, 16 heads: 346 -> 340 us;
+// depend on it, and no block needs its maximum first (below).  64 x 1,024 tokens, 16 heads: 344 -> 337 us;
 // the ragged 32-request batch's attention gains more (the 128-query workgroups leave no idle waves):
-// 4.96 -> 4.88 ms per forward.  What bounds it now is power: copies without the loads run 291 us, and
-// the MFMA stream alone lowers the clock to 1.6 GHz (19.6 ns per 32x32x16, 161 us in all).
+// 4.96 -> 4.88 ms per forward.  Counters at 64 x 1,024 tokens: VALU instructions take 57% of the SIMD cycles
+// and the matrix cores are busy 44%, so the two still run mostly one after the other, at 1.86 GHz where a
+// kernel without MFMAs runs at 2.43; copies without the loads run 291 us.
 template <typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void attention_ahead_kernel(AttnArgs a) {
   typedef typename Vec8<T>::type T8;

@@ -225,8 +225,8 @@ int laya_op_linear(const void* x, const void* w, const float* bias, void* out, i
                    int dtype16, int M, int N, int K, int splits, int tile, void* stream);
 
 /* The launch that tile -1 (or -2) stands for: *planned_tile and *planned_splits for laya_op_linear of
- * this kind (biased: with a bias), or for laya_op_qkv with N = 3 width, K = width (kind 5; 6 with RoPE).
- * Host arithmetic only: needs no device. */
+ * this kind (biased: with a bias), or for laya_op_qkv with N = 3 width, K = width (kind 5; 6 with RoPE); with
+ * tile -3 the launch that a laya_predict slot of M rows takes.  Host arithmetic only: needs no device. */
 int laya_op_plan(int kind, int dtype16, int M, int N, int K, int biased, int tile, int* planned_tile,
                  int* planned_splits);
 

@@ -37,6 +37,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <type_traits>
 
 namespace laya {
@@ -1561,19 +1562,21 @@ namespace {
 // gets, nk its 64-deep slabs per tile, R the rounds of workgroups (two per CU where LDS allows) and MB
 // the output's megabytes, with an own rate for fp32 output (o32) and an addition for RoPE (p).  Where the
 // tile count is no multiple of the 8 XCDs the tiles are walked row by row across them, and each of the
-// tile columns fetches A into another L2: q per megabyte of A, at most 8 times.
+// tile columns fetches A into another L2: q per megabyte of A, at most 8 times, over the root of L (more
+// rounds hide more of it).
 // Up to 512 rows the constants are fits to graph replays over weights that are cold in every cache (14
-// projections of widths 768 and 1,024 at 12 row counts).  Above, they are fits to the stage times of each
-// tile inside whole forwards of three encoders at 21 to 31 row classes and to replays of 700 problems
-// of random kind, depth and row count (tune_gemm_costs.py and its data): replays alone rank the tiles
-// otherwise than a forward does (constants fitted to them chose 128x256 tiles for down projections that
-// run 17% slower in it).  How far the choice is from the best tile measured, on average: 0.5% on 117
-// other replayed problems up to 512 rows; above, 0.9% on row classes and 0.7% on problems that were left out
-// of a fit made for that check, worst 14%.  Constants without q, o32 and p, fitted to replays at 18 row
-// counts, were 1.6% and 4.2% off, worst 24% and 35% (7,825 x 768 x 1,152 32.4 us against 24.4 by the
-// plan table and heuristic before them, 25.7 now; 15,104 x 768 x 768 in a forward 29.9 against 24.2 now), and
-// the table and heuristic 20-27% (us: 96-row QKV 6.6 -> 4.7, with RoPE 9.9 -> 4.9; 1,008-row GeGLU up
-// 14.1 -> 9.1).
+// projections of widths 768 and 1,024 at 12 row counts).  Above, a slot's plans and an op-level call's
+// have constants of their own, because the same launch takes other times: in a forward A was written by the
+// launch before (7,168 x 1,024 x 1,024 on tile 25: 22.3 us), a call that reads it from memory waits for it
+// (7,881 rows: 26-27 us, and the 256-row tile takes 23).  kForwardCosts are fits to the stage times of each tile
+// inside whole forwards of three encoders at 21 to 31 row classes, kReplayCosts to replays of 1,000 problems
+// of random kind, depth and row count (tune_gemm_costs.py and its data).  How far the choice is from the
+// best tile measured, on average, on row classes and problems left out of a fit made for that check: 0.5%
+// in forwards (worst 9%) and 0.4% in replays (worst 10%); on 117 replays up to 512 rows 0.5%.  One table of
+// constants without q, o32 and p, fitted to replays at 18 row counts, was 1.5% and 4.2% off, worst 24% and
+// 35% (15,104 x 768 x 768 in a forward 29.9 us against 24.2 now; 7,825 x 768 x 1,152 replayed 32.4 against 24.5),
+// one fitted to both 0.9% each, and the plan table and heuristic before them 20-27% in replays (us: 96-row QKV
+// 6.6 -> 4.7, with RoPE 9.9 -> 4.9; 1,008-row GeGLU up 14.1 -> 9.1).
 // An fp32 split costs its consumer another partial to read (0.12 us per 512 rows), and splits stop where
 // the partials would pass 16 MB.  Tile 33 has no row: no problem was found where the fit would choose it (it
 // remains for callers that name it).
@@ -1596,18 +1599,31 @@ constexpr TileCost kFewRowCosts[] = {
 };
 // Tile 21's two-stage pipeline falls behind with depth (15,088 x 768: 26.5 against the ring's 24.2 us at
 // K = 768 but 92 against 76 at 3,072), so it is kept to 16 slabs.
-constexpr TileCost kCosts[] = {
-    {14, 1, 3.108f, 0.204f, 0.919f, 0.644f, 0.320f, 0.027f, 0.f},
-    {31, 1, 2.083f, 0.257f, 0.716f, 0.785f, 0.336f, 0.f, 0.164f},
-    {34, 1, 2.110f, 0.430f, 1.189f, 0.486f, 0.178f, 0.f, 0.055f},
-    {23, 1, 2.924f, 0.309f, 0.712f, 0.443f, 0.247f, 0.015f, 0.f},
-    {24, 1, 2.879f, 0.311f, 0.604f, 0.482f, 0.251f, 0.013f, 0.f},
-    {25, 1, 2.776f, 0.450f, 0.159f, 0.504f, 0.247f, 0.015f, 0.113f},
-    {18, 1, 3.346f, 0.452f, 0.662f, 0.430f, 0.220f, 0.016f, 0.145f},
-    {9, 1, 3.938f, 0.972f, 0.415f, 0.354f, 0.155f, 0.013f, 0.089f},
-    {8, 1, 3.871f, 0.954f, 0.959f, 0.323f, 0.145f, 0.017f, 0.097f},
-    {21, 1, 5.205f, 1.065f, 2.073f, 0.347f, 0.121f, 0.013f, 0.f, 16},
-    {35, 1, 6.335f, 1.098f, 4.732f, 0.245f, 0.f, 0.002f, 0.299f},
+constexpr TileCost kForwardCosts[] = {
+    {14, 1, 2.950f, 0.200f, 0.678f, 0.737f, 0.376f, 0.f, 0.f},
+    {31, 1, 1.723f, 0.260f, 0.551f, 0.856f, 0.395f, 0.f, 0.144f},
+    {34, 1, 1.890f, 0.434f, 1.228f, 0.499f, 0.189f, 0.f, 0.044f},
+    {23, 1, 2.762f, 0.314f, 0.473f, 0.451f, 0.267f, 0.007f, 0.f},
+    {24, 1, 2.798f, 0.315f, 0.409f, 0.469f, 0.261f, 0.f, 0.f},
+    {25, 1, 2.810f, 0.459f, 0.114f, 0.452f, 0.238f, 0.011f, 0.071f},
+    {18, 1, 3.405f, 0.465f, 0.562f, 0.388f, 0.212f, 0.012f, 0.106f},
+    {9, 1, 3.931f, 1.016f, 0.f, 0.347f, 0.154f, 0.005f, 0.083f},
+    {8, 1, 3.748f, 0.984f, 0.452f, 0.328f, 0.145f, 0.014f, 0.082f},
+    {21, 1, 5.223f, 1.071f, 1.511f, 0.350f, 0.117f, 0.019f, 0.f, 16},
+    {35, 1, 5.968f, 1.125f, 4.160f, 0.235f, 0.f, 0.f, 0.285f},
+};
+constexpr TileCost kReplayCosts[] = {
+    {14, 1, 3.409f, 0.218f, 1.331f, 0.445f, 0.218f, 0.017f, 0.f},
+    {31, 1, 2.896f, 0.247f, 1.119f, 0.631f, 0.215f, 0.f, 0.185f},
+    {34, 1, 2.673f, 0.419f, 1.296f, 0.440f, 0.147f, 0.f, 0.088f},
+    {23, 1, 3.428f, 0.301f, 1.353f, 0.365f, 0.178f, 0.036f, 0.f},
+    {24, 1, 3.338f, 0.307f, 1.348f, 0.395f, 0.177f, 0.035f, 0.f},
+    {25, 1, 2.810f, 0.424f, 0.135f, 0.636f, 0.265f, 0.030f, 0.118f},
+    {18, 1, 3.336f, 0.422f, 0.825f, 0.529f, 0.225f, 0.027f, 0.158f},
+    {9, 1, 4.522f, 0.867f, 2.047f, 0.356f, 0.123f, 0.026f, 0.109f},
+    {8, 1, 4.376f, 0.881f, 1.909f, 0.335f, 0.127f, 0.025f, 0.119f},
+    {21, 1, 5.551f, 1.031f, 3.483f, 0.333f, 0.108f, 0.f, 0.f, 16},
+    {35, 1, 7.134f, 1.034f, 4.761f, 0.285f, 0.f, 0.005f, 0.302f},
 };
 
 template <size_t C>
@@ -1627,9 +1643,11 @@ bool cost_plan(const TileCost (&costs)[C], int M, int N, int K, Epi epi, int cus
       const long long work = tiles * z, rounds = (work + cus * c.per_cu - 1) / (cus * c.per_cu);
       const float mb = static_cast<float>(M) * N * (epi == Epi::F32 ? 4 * z : 2) * 1e-6f;
       const float per_mb = epi == Epi::F32 ? c.o32 : rope ? c.o + c.p : c.o;
+      const long long most = (work + cus - 1) / cus;
       const float a_mb = work % 8 ? static_cast<float>(std::min(8, N / d.bn)) * M * K * 2e-6f : 0.f;
-      const float t = c.a + c.s * static_cast<float>((work + cus - 1) / cus * ((nk + z - 1) / z)) +
-                      c.r * static_cast<float>(rounds - 1) + per_mb * mb + c.q * a_mb +
+      const float t = c.a + c.s * static_cast<float>(most * ((nk + z - 1) / z)) +
+                      c.r * static_cast<float>(rounds - 1) + per_mb * mb +
+                      c.q * a_mb / std::sqrt(static_cast<float>(most)) +
                       (epi == Epi::F32 ? 0.12f * z * static_cast<float>(std::max(M, 512)) / 512.f : 0.f);
       if (best < 0.f || t < best) {
         best = t;
@@ -1644,10 +1662,11 @@ bool cost_plan(const TileCost (&costs)[C], int M, int N, int K, Epi epi, int cus
 }  // namespace
 
 void gemm_plan(int M, int N, int K, Epi epi, DType t, int cus, int* tile, int* splits, bool rope, bool measured,
-               bool by_cost, int max_splits) {
-  if (by_cost && N % 64 == 0 && K >= kCostDepth &&
-      (M <= kFewRows ? cost_plan(kFewRowCosts, M, N, K, epi, cus, rope, max_splits, tile, splits)
-                     : cost_plan(kCosts, M, N, K, epi, cus, rope, max_splits, tile, splits)))
+               GemmCosts costs, int max_splits) {
+  if (costs != GemmCosts::None && N % 64 == 0 && K >= kCostDepth &&
+      (M <= kFewRows                   ? cost_plan(kFewRowCosts, M, N, K, epi, cus, rope, max_splits, tile, splits)
+       : costs == GemmCosts::Forward ? cost_plan(kForwardCosts, M, N, K, epi, cus, rope, max_splits, tile, splits)
+                                       : cost_plan(kReplayCosts, M, N, K, epi, cus, rope, max_splits, tile, splits)))
     return;
   for (const PlanEntry& e : kPlans) {
     if (!measured) break;

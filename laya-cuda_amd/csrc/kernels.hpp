@@ -80,12 +80,14 @@ GemmTile gemm_tile(int id);
 // Packed rows from which a problem counts as batched: the heuristic costs tiles by their operand
 // bytes per CU, and shape slots keep the out/down projections as 16-bit rows (no split-K).
 constexpr int kBatchedRows = 4096;
-// Chooses a tile and split count for a problem on `cus` compute units: the cost model
-// when `by_cost` and K is in its range, else the measured plan table (gemm_plans.inc) when it has the
-// problem and `measured`, else the heuristic.  At most `max_splits` splits (the cost model's choice only).
+// Whose times the planner's cost model takes: none, those of a call on its own, those inside a forward.
+enum class GemmCosts { None, Replay, Forward };
+// Chooses a tile and split count for a problem on `cus` compute units: the cost model when `costs` names
+// one and K is in its range, else the measured plan table (gemm_plans.inc) when it has the problem and
+// `measured`, else the heuristic.  At most `max_splits` splits (the cost model's choice only).
 // rope: the QKV epilogue applies RoPE, which needs wave tiles of 64-column multiples.
-void gemm_plan(int M, int N, int K, Epi epi, DType t, int cus, int* tile, int* splits, bool rope = false,
-               bool measured = true, bool by_cost = true, int max_splits = 8);
+void gemm_plan(int M, int N, int K, Epi epi, DType t, int cus, int* tile, int* splits, bool rope, bool measured,
+               GemmCosts costs, int max_splits = 8);
 hipError_t gemm_prepare();  // sets LDS attributes of the large-tile kernels (call once per device)
 // Pipelined tiles read their operands through buffer resources with 32-bit byte offsets: true when
 // both operands ([M][lda] and [N][ldb] 16-bit) span fewer than 2^32 bytes.

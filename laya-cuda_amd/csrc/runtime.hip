@@ -325,7 +325,7 @@ void plan_slot(const Engine& E, Slot* s, int m, int b, int k, int max_splits = 8
   LAYA_REQUIRE(gemm_operands_addressable(m, std::max(f, 4 * d), std::max(3 * d, 4 * d), std::max(f, 4 * d)),
                "a shape class of " + std::to_string(m) + " packed rows exceeds the 4 GiB GEMM operand limit");
   auto plan = [&](int M, int N, int K, Epi epi, int* tile, int* splits, bool rope = false) {
-    gemm_plan(M, N, K, epi, E.mfma(), E.cus, tile, splits, rope, true, true, max_splits);
+    gemm_plan(M, N, K, epi, E.mfma(), E.cus, tile, splits, rope, true, GemmCosts::Forward, max_splits);
   };
   plan(m, 3 * d, d, Epi::QKV, &s->tile[0], &s->splits[0], E.modern);
   plan(m, d, d, Epi::F32, &s->tile[1], &s->splits[1]);
@@ -1387,11 +1387,14 @@ static Epi op_epilogue(int kind) {
   constexpr Epi kinds[] = {Epi::F32, Epi::HALF, Epi::GELU, Epi::RELU, Epi::GEGLU, Epi::QKV, Epi::QKV};
   return kinds[kind];
 }
-// The planner's launch for an op-level GEMM (tile -1, or -2: the heuristic alone).
+// The planner's launch for an op-level GEMM (tile -1, or -2: the heuristic alone) or, with tile -3, for a
+// forward's.
 static void plan_op(int kind, int dtype16, int M, int N, int K, bool biased, int* tile, int* splits) {
-  // fp32 plans: the caller sums the split partials, so their number is the table's and heuristic's.
-  const bool planned = *tile == -1;
-  gemm_plan(M, N, K, op_epilogue(kind), half_type(dtype16), 256, tile, splits, kind == 6, planned, planned && kind != 0);
+  // Op-level fp32 plans: the caller sums the split partials, so their number is the table's and heuristic's.
+  const GemmCosts costs = *tile == -3                ? GemmCosts::Forward
+                          : *tile == -1 && kind != 0 ? GemmCosts::Replay
+                                                     : GemmCosts::None;
+  gemm_plan(M, N, K, op_epilogue(kind), half_type(dtype16), 256, tile, splits, kind == 6, *tile != -2, costs);
   if (biased || kind >= 5) *splits = 1;
 }
 
@@ -1399,7 +1402,7 @@ int laya_op_plan(int kind, int dtype16, int M, int N, int K, int biased, int til
                  int* planned_splits) {
   return guarded(nullptr, [&] {
     LAYA_REQUIRE(kind >= 0 && kind <= 6, "kind must be 0-4 (laya_op_linear), 5 (laya_op_qkv) or 6 (with RoPE)");
-    LAYA_REQUIRE(tile == -1 || tile == -2, "tile must be -1 (the planner) or -2 (its heuristic)");
+    LAYA_REQUIRE(tile <= -1 && tile >= -3, "tile must be -1 (the planner), -2 (its heuristic) or -3 (a forward's plan)");
     LAYA_REQUIRE(M > 0 && N > 0 && K > 0 && planned_tile && planned_splits, "positive sizes and both outputs");
     int splits = 1;
     plan_op(kind, dtype16, M, N, K, biased != 0, &tile, &splits);
@@ -1415,6 +1418,7 @@ int laya_op_linear(const void* x, const void* w, const float* bias, void* out, i
     LAYA_REQUIRE(kind >= 0 && kind <= 4,
                  "kind must be 0 (fp32), 1 (16-bit), 2 (16-bit GELU), 3 (16-bit ReLU) or 4 (16-bit GeGLU)");
     const Epi epi = op_epilogue(kind);
+    if (tile < -1) tile = -2;
     if (tile < 0) plan_op(kind, dtype16, M, N, K, bias != nullptr, &tile, &splits);
     LAYA_REQUIRE(tile < gemm_tile_count(), "bad tile id");
     LAYA_REQUIRE(K % 64 == 0 && N % gemm_tile(tile).bn == 0, "K must be a multiple of 64 and N of the tile width");
@@ -1434,6 +1438,7 @@ int laya_op_qkv(const void* x, const void* w, const float* bias, void* q, void* 
     int splits = 1;
     const bool rope = rope_cos != nullptr;
     LAYA_REQUIRE(!rope || (rope_sin && positions), "RoPE needs cos, sin and positions");
+    if (tile < -1) tile = -2;
     if (tile < 0) plan_op(rope ? 6 : 5, dtype16, M, 3 * width, width, false, &tile, &splits);
     LAYA_REQUIRE(tile < gemm_tile_count(), "bad tile id");
     LAYA_REQUIRE(width % 64 == 0 && (3 * width) % gemm_tile(tile).bn == 0, "width does not fit the tile");

@@ -1,4 +1,4 @@
-"""The GEMM planner's cost constants above 512 rows (gemm.hip kCosts): sweep, fit and check.
+"""The GEMM planner's cost constants above 512 rows (gemm.hip kForwardCosts, kReplayCosts): sweep, fit and check.
 
     python laya-cuda_amd/csrc/tune_gemm_costs.py sweep --seed 31 --count 700 --out <file>   (on the GPU)
     python laya-cuda_amd/csrc/tune_gemm_costs.py fit                                        (anywhere)
@@ -30,7 +30,6 @@ TILES = {14: (64, 64, True), 31: (64, 64, False), 34: (128, 64, False), 23: (128
          35: (256, 256, True)}
 NO_ROPE = (14, 23, 24, 21)  # wave tiles of less than a head
 CUS, MAX_SLABS = 256, {21: 16}
-FORWARD_WEIGHT = 3  # a forward's stage counts as much as three isolated launches
 
 
 def problems(seed, count):
@@ -126,7 +125,8 @@ def features(tile, M, N, K, splits, kind):
     rounds, mb = -(-work // CUS), M * N * (4 * splits if kind == "f32" else 2) * 1e-6
     f32 = kind == "f32"
     return [1, rounds * -(-(K // 64) // splits), rounds - 1, 0 if f32 else mb, mb if f32 else 0,
-            min(8, N // bn) * M * K * 2e-6 if across and work % 8 else 0, mb if kind == "rope" else 0]
+            min(8, N // bn) * M * K * 2e-6 / math.sqrt(rounds) if across and work % 8 else 0,
+            mb if kind == "rope" else 0]
 
 
 def fit(data):
@@ -183,18 +183,14 @@ def main():
         return sweep(args)
     data = json.loads(gzip.decompress((HERE / "gemm_cost_data.json.gz").read_bytes()))
     forward, isolated, held = data["forward"], data["isolated"], data["held_out"]
-    first = [x for i, x in enumerate(forward) if i // 4 % 2 == 0]  # every other row class, four projections each
-    second = [x for i, x in enumerate(forward) if i // 4 % 2 == 1]
-    half = fit(first * FORWARD_WEIGHT + isolated)
-    print("fitted to every other row class and the isolated sweep:")
-    print("  the other row classes in forwards:", regret(half, second))
-    print("  the held-out sweep:", regret(half, held))
-    costs = fit(forward * FORWARD_WEIGHT + isolated + held)
-    print("fitted to everything:")
-    print("  forwards:", regret(costs, forward))
-    print("  isolated:", regret(costs, isolated + held))
-    for tile, cost in costs.items():
-        print("    {%d, 1, %s}," % (tile, ", ".join("%.3ff" % c for c in cost)))
+    half = fit([x for i, x in enumerate(forward) if i // 4 % 2 == 0])  # every other row class, four projections each
+    print("forwards, fitted to every other row class:", regret(half, [x for i, x in enumerate(forward) if i // 4 % 2]))
+    print("isolated, fitted to the first sweep:", regret(fit(isolated), held))
+    for name, rows in (("kForwardCosts", forward), ("kReplayCosts", isolated + held)):
+        costs = fit(rows)
+        print(f"{name}, fitted to everything:", regret(costs, rows))
+        for tile, cost in costs.items():
+            print("    {%d, 1, %s}," % (tile, ", ".join("%.3ff" % c for c in cost)))
 
 
 if __name__ == "__main__":

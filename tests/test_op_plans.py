@@ -33,7 +33,7 @@ def test_only_fp32_products_without_bias_split():
 def test_bad_plan_requests_are_refused():
     lib, t = _lib.load(), ct.c_int32()
     for args in [(7, _lib.F16, 16, 64, 64, 0, -1), (-1, _lib.F16, 16, 64, 64, 0, -1), (1, _lib.F16, 0, 64, 64, 0, -1),
-                 (1, _lib.F16, 16, 64, 64, 0, 3)]:
+                 (1, _lib.F16, 16, 64, 64, 0, 3), (1, _lib.F16, 16, 64, 64, 0, -4)]:
         assert lib.laya_op_plan(*args, ct.byref(t), ct.byref(t)) == _lib.EINVAL
     assert lib.laya_op_plan(1, _lib.F16, 16, 64, 64, 0, -1, None, None) == _lib.EINVAL
 
@@ -41,17 +41,19 @@ def test_bad_plan_requests_are_refused():
 DATA = Path(__file__).resolve().parents[1] / "laya-cuda_amd" / "csrc" / "gemm_cost_data.json.gz"
 
 
-@pytest.mark.parametrize("where,mean,most", [("forward", 1.01, 1.14), ("held_out", 1.01, 1.15), ("isolated", 1.01, 1.25)])
-def test_planned_tiles_are_near_the_best_measured(where, mean, most):
+@pytest.mark.parametrize("where,tile,mean,most", [("forward", -3, 1.01, 1.11), ("held_out", -1, 1.005, 1.12),
+                                                  ("isolated", -1, 1.006, 1.13)])
+def test_planned_tiles_are_near_the_best_measured(where, tile, mean, most):
     """The planner's choice for 16-bit products of more than 512 rows against the times that its constants come
-    from (measured inside forwards and as isolated launches).  The bounds are what the constants reach:
-    mean 1.008, 1.007 and 1.009, largest 1.134, 1.145 and 1.239."""
+    from: inside forwards for a forward's plans, isolated launches for an op-level call's.  The bounds are what
+    the constants reach."""
     kinds = {"half": 1, "gelu": 2, "relu": 3, "geglu": 4, "qkv": 5, "rope": 6}
     ratios = []
     for kind, M, N, K, timed in json.loads(gzip.decompress(DATA.read_bytes()))[where]:
         if M > 512 and kind in kinds:
-            us = {tile: t for tile, _, t, _ in timed}
-            ratios.append(us[plan(kinds[kind], M, N, K)[0]] / min(us.values()))
+            us = {t: u for t, _, u, _ in timed}
+            ratios.append(us[plan(kinds[kind], M, N, K, tile=tile)[0]] / min(us.values()))
+    print(where, len(ratios), sum(ratios) / len(ratios), max(ratios))
     assert len(ratios) > 100
     assert sum(ratios) / len(ratios) <= mean and max(ratios) <= most
 
